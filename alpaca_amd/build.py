@@ -33,7 +33,7 @@ SOURCES += [(src, os.path.splitext(src)[0], []) for src in
 # keeps those results where the VALU reads them (the AGPR form adds a
 # v_accvgpr_read / write per result register).
 SOURCES += [(src, os.path.splitext(src)[0], ["-mllvm", "-amdgpu-mfma-vgpr-form=1"])
-            for src in ("kernels_gemm.hip", "kernels_attention.hip")]
+            for src in ("kernels_gemm.hip", "kernels_gemm_small.hip", "kernels_attention.hip")]
 ARCH = "gfx950"
 # Packed FP32 instructions are disabled: hipcc -O3 otherwise emits v_pk_* forms.
 FLAGS = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall", "-Wno-unused-function",

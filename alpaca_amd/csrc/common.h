@@ -311,6 +311,25 @@ struct QkvRope {
 // one-term before lo_row0 and k, v two-term throughout).
 hipError_t launch_gemm_qkv_rope(const f16* x, const f16* xlo, int ldx, int m, const DevMatrix& w, const QkvRope& o,
                                 hipStream_t st, int lo_row0 = 0, int lo_out_row0 = 0, int lo_col0 = 1 << 30);
+// The same products for few rows (kernels_gemm_small.hip), K split over the
+// waves of a workgroup; hipErrorNotSupported where the shapes do not fit or the
+// pipelined tiles are faster.  The input is the activations' f16 terms (x,
+// xlo) or, with `gain` set, the float32 rows xf (row stride ldx), RMS-normalised
+// on the way in and rounded to the same terms (second terms as lo_row0 /
+// lo_col0 say; a lo_row0 past the last row: none).  `rope` for GEMM_QKV_ROPE.
+// launch_gemm_mfma and launch_gemm_qkv_rope take it where it applies.
+struct SmallGemmInput {
+    const f16* x = nullptr;
+    const f16* xlo = nullptr;
+    const float* xf = nullptr;
+    const float* gain = nullptr;
+    float eps = 0.f;
+    int ldx = 0;
+};
+bool gemm_small_takes(const SmallGemmInput& in, int m, const DevMatrix& w, const DevMatrix* w_up);
+hipError_t launch_gemm_small(const SmallGemmInput& in, int m, const DevMatrix& w, const DevMatrix* w_up, float* y,
+                             f16* yh, f16* yhlo, int ldy, int mode, const QkvRope* rope, hipStream_t st, int lo_row0,
+                             int lo_out_row0, int lo_col0 = 1 << 30);
 // exact: x f32; float32 FMA in the reference's per-block order.  SWIGLU writes y f32.
 hipError_t launch_gemm_f32(const float* x, int ldx, int m, const DevMatrix& w, const DevMatrix* w_up, float* y,
                            int ldy, int mode, hipStream_t st);

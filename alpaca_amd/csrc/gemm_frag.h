@@ -1,0 +1,22 @@
+// Quants to exact f16 MFMA fragments, shared by the prefill GEMMs.
+#pragma once
+
+#include "common.h"
+
+typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
+__device__ __forceinline__ uint32_t as_u32(h2 v) { return __builtin_bit_cast(uint32_t, v); }
+
+// 4 signed bytes -> 2 dwords holding the 4 quants as f16 pairs (exact).
+__device__ __forceinline__ void int8x4_to_f16(uint32_t w, uint32_t& o0, uint32_t& o1) {
+    const uint32_t u = w ^ 0x80808080u;  // q + 128 in each byte
+    const h2 bias = {(f16)1152.0f, (f16)1152.0f};
+    o0 = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) - bias);
+    o1 = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) - bias);
+}
+// 4 nibbles (one per byte, already masked) -> nib - 8 as f16 pairs (exact).
+__device__ __forceinline__ void nib4_to_f16(uint32_t nib, uint32_t& o0, uint32_t& o1) {
+    const h2 bias = {(f16)1032.0f, (f16)1032.0f};
+    o0 = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, nib, 0x04010400u)) - bias);
+    o1 = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, nib, 0x04030402u)) - bias);
+}

@@ -18,7 +18,8 @@
 // tensor-op path does moves C1 prefill logits past the 2e-3 bound against the
 // CPU reference; single-term activations keep C1 inside it but not the larger
 // configurations.)
-//   dgemm_kernel: global -> LDS DMA, three stages in flight (the default).
+//   dgemm_kernel: global -> LDS DMA, three stages in flight (the default;
+//   grids of few rows go to kernels_gemm_small.hip).
 //   gemm_mfma_kernel: register-staged, double-buffered; shapes the DMA kernel
 //   does not take.
 // Epilogues: store f32, accumulate into the f32 residual, or SwiGLU
@@ -29,6 +30,7 @@
 // block sum is scaled once (acc += d * s), with FP contraction off, so each
 // output equals the CPU reference's float32 result.
 #include "common.h"
+#include "gemm_frag.h"
 
 #include <type_traits>
 
@@ -525,24 +527,6 @@ hipError_t launch_gemm_f32(const float* x, int ldx, int m, const DevMatrix& w, c
 // (1024 + q + 128) - 1152 = q exactly).  Tiles are taken in an XCD-major
 // order so that tiles sharing A rows run on one XCD and share its L2.
 namespace {
-
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-__device__ __forceinline__ h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
-__device__ __forceinline__ uint32_t as_u32(h2 v) { return __builtin_bit_cast(uint32_t, v); }
-
-// 4 signed bytes -> 2 dwords holding the 4 quants as f16 pairs (exact).
-__device__ __forceinline__ void int8x4_to_f16(uint32_t w, uint32_t& o0, uint32_t& o1) {
-    const uint32_t u = w ^ 0x80808080u;  // q + 128 in each byte
-    const h2 bias = {(f16)1152.0f, (f16)1152.0f};
-    o0 = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04010400u)) - bias);
-    o1 = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, u, 0x04030402u)) - bias);
-}
-// 4 nibbles (one per byte, already masked) -> nib - 8 as f16 pairs (exact).
-__device__ __forceinline__ void nib4_to_f16(uint32_t nib, uint32_t& o0, uint32_t& o1) {
-    const h2 bias = {(f16)1032.0f, (f16)1032.0f};
-    o0 = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, nib, 0x04010400u)) - bias);
-    o1 = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, nib, 0x04030402u)) - bias);
-}
 
 constexpr int DBK = 64;  // K per stage
 
@@ -1351,6 +1335,15 @@ hipError_t launch_gemm_mfma(const f16* x, const f16* xlo, int ldx, int m, const 
     if (w.cols % DBK || ldx % 8 || ((uintptr_t)x & 15) || ((uintptr_t)xlo & 15) ||
         (quant && (!w.s2 || (w_up && !w_up->s2))) || !dma_offsets_fit(m, ldx, w))
         return launch_gemm_mfma_staged(x, xlo, ldx, m, w, w_up, y, yh, yhlo, ldy, mode, st, lo_row0, lo_out_row0);
+    {
+        SmallGemmInput in;
+        in.x = x;
+        in.xlo = xlo;
+        in.ldx = ldx;
+        const hipError_t e =
+            launch_gemm_small(in, m, w, w_up, y, yh, yhlo, ldy, mode, nullptr, st, lo_row0, lo_out_row0);
+        if (e != hipErrorNotSupported) return e;
+    }
     GemmArgs a;
     a.x = x;
     a.xlo = xlo;
@@ -1382,6 +1375,15 @@ hipError_t launch_gemm_qkv_rope(const f16* x, const f16* xlo, int ldx, int m, co
         o.hd > 128 || o.heads <= 0 || o.kv_heads <= 0 || w.rows != (o.heads + 2 * o.kv_heads) * o.hd || !o.rope ||
         !o.qh || !o.kc || !o.vc)
         return hipErrorNotSupported;
+    {
+        SmallGemmInput in;
+        in.x = x;
+        in.xlo = xlo;
+        in.ldx = ldx;
+        const hipError_t e = launch_gemm_small(in, m, w, nullptr, nullptr, o.qh, o.qlo, o.heads * o.hd, GEMM_QKV_ROPE,
+                                               &o, st, lo_row0, lo_out_row0, lo_col0);
+        if (e != hipErrorNotSupported) return e;
+    }
     GemmArgs a;
     a.x = x;
     a.xlo = xlo;

@@ -1376,8 +1376,12 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
     // and 64-query blocks then either lie wholly in that range or wholly
     // before it, so the same rows take two terms whatever tile a GEMM picks.
     // With lo_all_rows every row takes them.
-    const int lo = s->two_term ? s->lo_terms : 0;
-    const bool all = s->lo_all_rows;
+    // Below 16 rows every operand of every session takes its second term: such
+    // a call's activations keep float32 grade whatever the session's precision
+    // (one MFMA tile of rows costs the same with one term or two).
+    const bool few = n < 16;
+    const int lo = few ? kLoAll : s->two_term ? s->lo_terms : 0;
+    const bool all = s->lo_all_rows || few;
     const int tail0 = all ? 0 : last ? (n - 1) / 256 * 256 : n;
     const int lo_tile = tail0;
     auto want = [&](int bit) { return (lo & bit) && (all || last); };
@@ -1388,13 +1392,23 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
     f16* ffnhlo = want(kLoDown) ? s->ffnh.as<f16>() + B * F + r * F : nullptr;
     const int p_terms = want(kLoP) ? 2 : 1;
     float* ctx = s->ctx.as<float>() + r * QW;
-    s->stage("rmsnorm");
-    LAUNCH(launch_rmsnorm(x, L.attn_norm.as<float>(), nullptr, xh, xhlo_qkv, n, H, c.rms_norm_eps, st));
-    s->stage("qkv projections");
+    // Few rows: the RMSNorm runs inside the QKV and gate/up GEMMs where
+    // gemm_small_takes says so.
+    auto normed_row = [&](const DevBuf& gain) {
+        SmallGemmInput in;
+        in.xf = x;
+        in.gain = gain.as<float>();
+        in.eps = c.rms_norm_eps;
+        in.ldx = H;
+        return in;
+    };
+    const int none = 1 << 30;  // a first row past the last: no second terms
+    const DevMatrix& wqkv = L.pre(L.qkv, L.qkv16);
     hipError_t fused = hipErrorNotSupported;
-    if (flash && s->fuse_qkv_rope) {
+    const bool rope_fused = flash && s->fuse_qkv_rope;
+    QkvRope o;
+    if (rope_fused) {
         // RoPE and the KV append in the GEMM epilogue (q/k/v never reach HBM as f32)
-        QkvRope o;
         o.rope = rope;
         o.qh = qh;
         o.qlo = qhlo;
@@ -1405,16 +1419,34 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
         o.hd = hd;
         o.pos = pos;
         o.capacity = s->capacity;
-        // k and v take the second term on every row; q too unless ALPACA_HIP_QKV_LO=kv (read at
-        // session creation), which keeps it to the tail rows: 1% faster at the 1.7B shape, and
-        // the 135M shape's logit error 0.13 -> 0.20 of the bound, so it is off by default
-        fused = launch_gemm_qkv_rope(xh, xhlo_qkv, H, n, L.pre(L.qkv, L.qkv16), o, st, s->qkv_lo_all ? 0 : tail0,
-                                     tail0, s->qkv_lo_all ? 0 : QW);
-        if (fused != hipErrorNotSupported) LAUNCH(fused);
+    }
+    // k and v take the second term on every row; q too unless ALPACA_HIP_QKV_LO=kv (read at
+    // session creation), which keeps it to the tail rows: 1% faster at the 1.7B shape, and
+    // the 135M shape's logit error 0.13 -> 0.20 of the bound, so it is off by default
+    const int qkv_lo0 = s->qkv_lo_all ? 0 : tail0, qkv_col0 = s->qkv_lo_all ? 0 : QW;
+    const SmallGemmInput qkv_in = normed_row(L.attn_norm);
+    if (gemm_small_takes(qkv_in, n, wqkv, nullptr)) {
+        s->stage("qkv projections");
+        if (rope_fused) {
+            fused = launch_gemm_small(qkv_in, n, wqkv, nullptr, nullptr, o.qh, o.qlo, QW, GEMM_QKV_ROPE, &o, st,
+                                      xhlo_qkv ? qkv_lo0 : none, tail0, xhlo_qkv ? qkv_col0 : none);
+            LAUNCH(fused);
+        } else {
+            LAUNCH(launch_gemm_small(qkv_in, n, wqkv, nullptr, qkv, nullptr, nullptr, LDQKV, GEMM_STORE, nullptr, st,
+                                     xhlo_qkv ? 0 : none, 0));
+        }
+    } else {
+        s->stage("rmsnorm");
+        LAUNCH(launch_rmsnorm(x, L.attn_norm.as<float>(), nullptr, xh, xhlo_qkv, n, H, c.rms_norm_eps, st));
+        s->stage("qkv projections");
+        if (rope_fused) {
+            fused = launch_gemm_qkv_rope(xh, xhlo_qkv, H, n, wqkv, o, st, qkv_lo0, tail0, qkv_col0);
+            if (fused != hipErrorNotSupported) LAUNCH(fused);
+        }
+        if (fused == hipErrorNotSupported)
+            LAUNCH(launch_gemm_mfma(xh, xhlo_qkv, H, n, wqkv, nullptr, qkv, nullptr, nullptr, LDQKV, GEMM_STORE, st));
     }
     if (fused == hipErrorNotSupported) {
-        LAUNCH(launch_gemm_mfma(xh, xhlo_qkv, H, n, L.pre(L.qkv, L.qkv16), nullptr, qkv, nullptr, nullptr, LDQKV,
-                                GEMM_STORE, st));
         s->stage("rope + kv store");
         LAUNCH(launch_rope_store(qkv, LDQKV, n, c.head_count, c.kv_head_count, hd, pos, rope, 1, flash ? 0 : 1,
                                  flash ? qh : nullptr, flash ? qhlo : nullptr, kc, vc, s->kv_f16, s->capacity, st));
@@ -1462,11 +1494,19 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
     } else {
         LAUNCH(launch_gemm_mfma(ctxh, ctxhlo, QW, n, wo, nullptr, x, nullptr, nullptr, H, GEMM_ACC, st, lo_tile));
     }
-    s->stage("rmsnorm");
-    LAUNCH(launch_rmsnorm(x, L.ffn_norm.as<float>(), nullptr, xh, xhlo_ffn, n, H, c.rms_norm_eps, st, tail0));
-    s->stage("ffn gate+up+silu");
     const DevMatrix &wg = L.pre(L.gate, L.gate16), &wu = L.pre(L.up, L.up16);
-    if ((side & kSideGateUp) && xhlo_ffn && ffnhlo) {
+    const bool side_gu = (side & kSideGateUp) && xhlo_ffn && ffnhlo;
+    const SmallGemmInput ffn_in = normed_row(L.ffn_norm);
+    const bool ffn_normed = !side_gu && gemm_small_takes(ffn_in, n, wg, &wu);
+    if (!ffn_normed) {
+        s->stage("rmsnorm");
+        LAUNCH(launch_rmsnorm(x, L.ffn_norm.as<float>(), nullptr, xh, xhlo_ffn, n, H, c.rms_norm_eps, st, tail0));
+    }
+    s->stage("ffn gate+up+silu");
+    if (ffn_normed) {
+        LAUNCH(launch_gemm_small(ffn_in, n, wg, &wu, nullptr, ffnh, ffnhlo, F, GEMM_SWIGLU, nullptr, st,
+                                 xhlo_ffn ? lo_tile : none, tail0));
+    } else if (side_gu) {
         LAUNCH(launch_gemm_mfma(xh, nullptr, H, n - 1, wg, &wu, nullptr, ffnh, ffnhlo, F, GEMM_SWIGLU, st, 0, tail0));
         LAUNCH(launch_gemv_pair(wg, &wu, xh + lr * H, xhlo_ffn + lr * H, nullptr, ffnh + lr * F, ffnhlo + lr * F,
                                 GEMV_SWIGLU, st));
@@ -1570,8 +1610,11 @@ static int encode_chunk(ahip_session* s, const int32_t* dtok, int n, int pos, bo
     float* x = s->x.as<float>();
     float* qkv = s->qkv.as<float>();
     const float2* rope = m->rope.as<float2>();
-    const bool mfma = s->fast && n >= 16 && !s->prefill_f32_gemm;
-    const bool flash = s->fast && n >= 16 && !s->prefill_generic_attention && s->kv_f16 && (hd == 64 || hd == 128);
+    const bool flash_fits = s->fast && !s->prefill_generic_attention && s->kv_f16 && (hd == 64 || hd == 128);
+    // (below 16 rows every operand takes its second term, encode_mfma_layer; without the flash
+    // kernel those calls stay on the float32 kernels)
+    const bool mfma = s->fast && !s->prefill_f32_gemm && (n >= 16 || flash_fits);
+    const bool flash = flash_fits && (n >= 16 || mfma);
     if (mfma && n >= env_int("ALPACA_HIP_SPLIT_MIN", kSplitPrefillMin) && !s->profiling && env_int("ALPACA_HIP_PREFILL_STREAMS", 2) >= 2 &&
         prefill_split_pays(n, QW + 2 * KW)) {
         if (!s->part_stream[1]) s->part_stream[1] = split_stream_acquire(m->device);
