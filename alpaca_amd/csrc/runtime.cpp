@@ -1893,7 +1893,7 @@ static int run_sample(const float* dlogits, int n, float temperature, int top_k,
     if (!idx.p)
         if (int rc = idx.alloc((size_t)n * 4)) return rc;
     if (!prob.p)
-        if (int rc = prob.alloc((size_t)n * 8)) return rc;
+        if (int rc = prob.alloc(sample_scratch_bytes(n))) return rc;
     if (!out.p)
         if (int rc = out.alloc(8)) return rc;
     LAUNCH(launch_sample(dlogits, n, temperature, top_k, top_p, u, out.as<int32_t>(), out.as<int>() + 1,

@@ -153,3 +153,38 @@ def test_session_sampling_reads_the_last_logits(hip_ctx, hip_ops):
         toks.append(sampler.sample(s))
         s.decode(toks[-1])
     assert all(0 <= t < spec.config.vocab_size for t in toks)
+
+
+def edge_logits(n, kind):
+    rng = np.random.default_rng(n + len(kind))
+    l = (rng.standard_normal(n) * 3).astype(np.float32)
+    if kind == "equal":  # more ties than a window holds: no threshold separates them
+        l[:] = 0.25
+    elif kind == "steps":  # two values, the larger on every third
+        l[:] = 0.0
+        l[::3] = 2.0
+    elif kind == "inf":
+        l[::2] = -np.inf
+    return l
+
+
+@pytest.mark.parametrize("n", [1, 63, 65, 1024, 1025, 5000, 16385, 49153, 70000])
+@pytest.mark.parametrize("kind", ["normal", "equal", "steps", "inf"])
+def test_device_sampler_at_the_edges_of_its_runs(hip_ops, n, kind):
+    """Sizes around a run (1024 logits a workgroup), a maximum's 64, the logits held in registers
+    (16,384 and 49,152) and past them; ties past a window (1024 candidates), logits of -inf; top-k
+    and nuclei inside one window, at it and over several.  The largest draw, u = 1 - 2^-53, lies
+    within 2^-53 (1.1e-16, relative) of the end of the last token's interval; without top-k and
+    top-p, where the sums are associated by run (about 1e-16), it is a draw at a boundary too."""
+    l = edge_logits(n, kind)
+    rng = np.random.default_rng(n)
+    for t, k, p in ((0.0, 0, 1.0), (0.8, 0, 1.0), (0.8, 40, 0.95), (1.0, 512, 1.0), (1.0, 1024, 0.9),
+                    (1.2, 2500, 0.99), (0.7, 0, 0.5), (1.3, 0, 0.97)):
+        for u in (*rng.random(3), 0.0, 1 - 2**-53):
+            if t > 0 and u + 1e-12 > 1 and (k == 0 or k >= n) and p == 1.0:
+                continue
+            want = orc.sample(l, t, k, p, u)
+            if t > 0 and (orc.sample(l, t, k, p, max(u - 1e-12, 0.0)) != want
+                          or orc.sample(l, t, k, p, min(u + 1e-12, 1 - 2**-53)) != want):
+                continue  # as above: a draw at a boundary between two tokens
+            assert hip_ops.sample(l, t, k, p, u) == want, (n, kind, t, k, p, u)
