@@ -713,6 +713,123 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(const float* q, int ld
     }
 }
 
+// Several queries in float32 (exact prefill, f32 cache, head dims the flash
+// kernel does not take): a workgroup takes 16 queries of one head, its four
+// waves every fourth tile of 16 keys, with online softmax states that merge in
+// LDS.  Products run on the float32 matrix instructions (f32 operands, f32
+// sums): S^T = K Q^T leaves lane (g, c) with the scores of keys 4g..4g+3 for
+// query c, which is the B operand of O^T += V^T P^T when its four keys of step
+// r are taken as {4g + r}, so no probability crosses lanes.  K's dims are
+// paired with Q's in the same permuted order (16 B of a row per lane).  The
+// generic kernel below walks one query per wave, a key per lane and then a key
+// at a time: 150 queries of the 135M shape 55 us -> 8.6.
+template <int HD, typename KV>
+__global__ __launch_bounds__(256) void attn_f32_kernel(const float* q, int ldq, const KV* kc, const KV* vc, int cap,
+                                                       int H, int KVH, int T, int start, float* out, float scale) {
+    constexpr int KC = HD / 16, DT = HD / 16;
+    __shared__ float xo[4][16][HD];  // partial outputs, [wave][query][dim]
+    __shared__ float xml[4][2][16];  // the waves' max and sum
+    const int h = blockIdx.x, t0 = blockIdx.y * 16, kvh = h / (H / KVH);
+    const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tq = min(t0 + c16, T - 1), pos = start + tq;
+    const int kend = start + min(t0 + 16, T);  // keys [0, kend) cover every query
+    const KV* kb = kc + (int64_t)kvh * cap * HD;
+    const KV* vb = vc + (int64_t)kvh * cap * HD;
+    auto load4 = [](const KV* p) {
+        if constexpr (sizeof(KV) == 4) {
+            return *(const f32x4*)p;
+        } else {
+            const f16x4 v = *(const f16x4*)p;
+            return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
+        }
+    };
+    f32x4 qv[KC];
+#pragma unroll
+    for (int c = 0; c < KC; c++) qv[c] = *(const f32x4*)(q + (int64_t)tq * ldq + h * HD + 16 * c + 4 * g);
+    f32x4 o[DT];
+#pragma unroll
+    for (int d = 0; d < DT; d++) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+    for (int k0 = wave * 16; k0 < kend; k0 += 64) {
+        // rows past the last key repeat it (masked below)
+        const KV* kr = kb + (int64_t)min(k0 + c16, kend - 1) * HD + 4 * g;
+        f32x4 kv[KC];
+#pragma unroll
+        for (int c = 0; c < KC; c++) kv[c] = load4(kr + 16 * c);
+        float vv[4][DT];
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            const KV* vr = vb + (int64_t)min(k0 + 4 * g + r, kend - 1) * HD + c16;
+#pragma unroll
+            for (int d = 0; d < DT; d++) vv[r][d] = (float)vr[16 * d];
+        }
+        f32x4 s = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int c = 0; c < KC; c++)
+#pragma unroll
+            for (int e = 0; e < 4; e++) s = __builtin_amdgcn_mfma_f32_16x16x4f32(kv[c][e], qv[c][e], s, 0, 0, 0);
+        float mx = -INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; r++) {
+            s[r] = k0 + 4 * g + r <= pos ? s[r] * scale : -INFINITY;
+            mx = fmaxf(mx, s[r]);
+        }
+        mx = xor32_combine(xor16_combine(mx, MaxOp()), MaxOp());
+        const float mn = fmaxf(m, mx), mref = mn == -INFINITY ? 0.f : mn;  // (no key of the query yet)
+        const float alpha = expf(m - mref);
+        f32x4 p;
+#pragma unroll
+        for (int r = 0; r < 4; r++) p[r] = expf(s[r] - mref);
+        const float ps = (p[0] + p[1]) + (p[2] + p[3]);
+        l = l * alpha + xor32_combine(xor16_combine(ps, AddOp()), AddOp());
+#pragma unroll
+        for (int d = 0; d < DT; d++) o[d] *= alpha;
+#pragma unroll
+        for (int r = 0; r < 4; r++)
+#pragma unroll
+            for (int d = 0; d < DT; d++) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[r][d], p[r], o[d], 0, 0, 0);
+        m = mn;
+    }
+    // o[d][r] = O(query c16, dim 16 d + 4 g + r)
+#pragma unroll
+    for (int d = 0; d < DT; d++) *(f32x4*)&xo[wave][c16][16 * d + 4 * g] = o[d];
+    if (g == 0) {
+        xml[wave][0][c16] = m;
+        xml[wave][1][c16] = l;
+    }
+    __syncthreads();
+    for (int i = threadIdx.x; i < 16 * HD; i += 256) {
+        const int qr = i / HD, d = i % HD;
+        if (t0 + qr >= T) break;
+        float mt = xml[0][0][qr];  // finite: the first wave saw key 0
+#pragma unroll
+        for (int w = 1; w < 4; w++) mt = fmaxf(mt, xml[w][0][qr]);
+        float lt = 0.f, ot = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; w++) {
+            const float a = expf(xml[w][0][qr] - mt);
+            lt += a * xml[w][1][qr];
+            ot += a * xo[w][qr][d];
+        }
+        out[((int64_t)(t0 + qr) * H + h) * HD + d] = ot / lt;
+    }
+}
+
+template <typename KV>
+bool run_attn_f32(int hd, dim3 grid, hipStream_t st, const float* q, int ldq, const void* kc, const void* vc, int cap,
+                  int H, int KVH, int T, int start, float* out, float scale) {
+    const KV* k = (const KV*)kc;
+    const KV* v = (const KV*)vc;
+    switch (hd) {
+    case 32: attn_f32_kernel<32, KV><<<grid, 256, 0, st>>>(q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
+    case 64: attn_f32_kernel<64, KV><<<grid, 256, 0, st>>>(q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
+    case 96: attn_f32_kernel<96, KV><<<grid, 256, 0, st>>>(q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
+    case 128: attn_f32_kernel<128, KV><<<grid, 256, 0, st>>>(q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
+    default: return false;
+    }
+}
+
 // Merges per-split (max, sum, unnormalised output) triples (at most 64
 // splits): the first wave takes one split per lane for the weights
 // exp(m_s - M) and the weighted sum of the row sums, so the splits' statistics
@@ -1210,6 +1327,16 @@ hipError_t launch_attention_generic(const float* q, int ldq, const void* kc, con
     int split_len = (max_len + splits - 1) / splits;
     split_len = (split_len + 63) / 64 * 64;
     const float scale = 1.0f / sqrtf((float)hd);
+    // several queries: tiles of 16 (rows of 16-byte alignment; head dims past 128
+    // would hold too many accumulators)
+    if (tokens > 1 && splits == 1 && !((uintptr_t)q & 15) && ldq % 4 == 0) {
+        const dim3 tiles(heads, (tokens + 15) / 16);
+        const bool took = kv_f16 ? run_attn_f32<f16>(hd, tiles, st, q, ldq, kc, vc, capacity, heads, kv_heads, tokens,
+                                                     start, out, scale)
+                                 : run_attn_f32<float>(hd, tiles, st, q, ldq, kc, vc, capacity, heads, kv_heads,
+                                                       tokens, start, out, scale);
+        if (took) return hipGetLastError();
+    }
     dim3 grid(splits, heads, tokens);
     if (kv_f16)
         attn_generic_kernel<f16><<<grid, 64, 0, st>>>(q, ldq, (const f16*)kc, (const f16*)vc, capacity, heads,

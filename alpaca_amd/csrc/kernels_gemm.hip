@@ -25,10 +25,10 @@
 // Epilogues: store f32, accumulate into the f32 residual, or SwiGLU
 // (silu(x Wg^T) * (x Wu^T) from two accumulator sets) written as f16.
 //
-// gemm_f32_kernel (exact): float32 SIMT tiles 64x64, BK = 32 = one block.
-// Inside a block the products are summed in the CPU reference's order and the
-// block sum is scaled once (acc += d * s), with FP contraction off, so each
-// output equals the CPU reference's float32 result.
+// gemm_f32_kernel (exact): float32 on the VALU.  Inside a block the products are
+// summed in the CPU reference's order and the block sum is scaled once
+// (acc += d * s), with FP contraction off, so each output equals the CPU
+// reference's float32 result.
 #include "common.h"
 #include "gemm_frag.h"
 
@@ -304,10 +304,6 @@ hipError_t pick_tile_terms(const GemmArgs& a, int mode, hipStream_t st) {
 }
 
 // ------------------------------------------------------------------ exact path
-constexpr int FB = 64;       // tile edge (tokens and rows)
-constexpr int FK = 32;       // one quant block per stage
-constexpr int FP = FB + 4;   // LDS pitch in floats
-
 struct GemmF32Args {
     const float* x;
     int ldx, M;
@@ -316,145 +312,256 @@ struct GemmF32Args {
     int ldy;
 };
 
-// Weight (row n, column k) as an unscaled value: q for Q8_0, nib-8 for Q4_0,
-// the f16 value for F16.  The block scale is applied once per block sum.
-template <int FMT>
-__device__ __forceinline__ float w_raw(const DevMatrix& m, int n, int k, int K) {
-    if (FMT == DT_Q8_0) return (float)((const int8_t*)m.q)[(int64_t)n * K + k];
-    if (FMT == DT_Q4_0) {
-        const int j = k & 31;
-        const uint8_t b = m.q[((int64_t)n * (K >> 5) + (k >> 5)) * 16 + (j & 15)];
-        return (float)((int)(j < 16 ? (b & 15) : (b >> 4)) - 8);
+// Wave-uniform activations by scalar loads: x was written by earlier kernels
+// and is not written by this one.
+typedef const __attribute__((address_space(4))) float* scalar_f32;
+
+// Epilogue of one output (row m, column n) from its sums.
+template <int MODE>
+__device__ __forceinline__ void f32_finish(const GemmF32Args& p, int m, int n, float acc0, float acc1) {
+#pragma clang fp contract(off)
+    const int64_t o = (int64_t)m * p.ldy + n;
+    if (MODE == GEMM_STORE) {
+        p.y[o] = acc0;
+    } else if (MODE == GEMM_ACC) {
+        p.y[o] = p.y[o] + acc0;
+    } else {
+        const float e = expf(-acc0);
+        const float den = 1.0f + e;
+        p.y[o] = (acc0 / den) * acc1;
     }
-    return (float)((const f16*)m.q)[(int64_t)n * K + k];
 }
 
-template <int FMT, int MODE>
-__global__ __launch_bounds__(256) void gemm_f32_kernel(GemmF32Args p) {
+// Quantised weights.  The reference's order fixes the sum inside a 32-weight
+// block and the order in which the scaled block sums are added, but blocks are
+// independent of each other: a workgroup's waves take one block each, and the
+// scaled sums meet in LDS, where one thread per output adds them in order (the
+// same bits as one thread walking K).  A lane owns a weight row (64 per wave),
+// so a block's quants are converted once for MT rows of activations, which are
+// wave-uniform and come as scalar operands: two VALU instructions per product
+// and nothing else, the least that separate roundings of product and sum allow.
+template <int FMT, int MODE, int MT>
+__global__ __launch_bounds__(1024) void gemm_f32_kernel(GemmF32Args p) {
 #pragma clang fp contract(off)
+    static_assert(FMT == DT_Q8_0 || FMT == DT_Q4_0, "quantised weights");
     constexpr int NB = MODE == GEMM_SWIGLU ? 2 : 1;
-    constexpr bool kQuant = FMT != DT_F16;
-    __shared__ float Xs[FK][FP];
-    __shared__ float Ws[NB][FK][FP];
-    __shared__ float Ds[NB][FB];
+    extern __shared__ __attribute__((aligned(16))) float parts[];  // [2][NW][NB * MT][64]
+    const int K = p.w.cols, N = p.w.rows, M = p.M, nb = K >> 5;
+    const int NW = blockDim.x >> 6, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = blockIdx.y * 64, m0 = blockIdx.x * MT, n = min(n0 + lane, N - 1);
+    const int phases = (nb + NW - 1) / NW;
+    scalar_f32 xr[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) xr[i] = (scalar_f32)(p.x + (int64_t)min(m0 + i, M - 1) * p.ldx);
 
-    const int K = p.w.cols, N = p.w.rows, M = p.M;
-    const int m0 = blockIdx.x * FB, n0 = blockIdx.y * FB;
-    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
-
-    float acc[NB][4][4];
+    // outputs o = thread, thread + 64 NW, ... of the workgroup's MT x 64
+    constexpr int kOwn = MT;  // (at NW = 1)
+    float acc[NB][kOwn];
 #pragma unroll
     for (int mat = 0; mat < NB; mat++)
 #pragma unroll
-        for (int i = 0; i < 4; i++)
-#pragma unroll
-            for (int j = 0; j < 4; j++) acc[mat][i][j] = 0.f;
+        for (int k = 0; k < kOwn; k++) acc[mat][k] = 0.f;
 
-    const int lr = tid >> 2, lk = (tid & 3) * 8;
-    for (int k0 = 0; k0 < K; k0 += FK) {
-        {
-            const int m = m0 + lr;
-#pragma unroll
-            for (int j = 0; j < 8; j++) Xs[lk + j][lr] = m < M ? p.x[(int64_t)m * p.ldx + k0 + lk + j] : 0.f;
-        }
+    int4 raw[NB][2];
+    float d[NB];
+    auto load = [&](int b) {
 #pragma unroll
         for (int mat = 0; mat < NB; mat++) {
             const DevMatrix& w = mat ? p.u : p.w;
-            const int n = n0 + lr;
-#pragma unroll
-            for (int j = 0; j < 8; j++) Ws[mat][lk + j][lr] = n < N ? w_raw<FMT>(w, n, k0 + lk + j, K) : 0.f;
-            if (kQuant && lk == 0) Ds[mat][lr] = n < N ? (float)w.s[(int64_t)n * (K >> 5) + (k0 >> 5)] : 0.f;
-        }
-        __syncthreads();
-        if (kQuant) {
-            float blk[NB][4][4];
-#pragma unroll
-            for (int mat = 0; mat < NB; mat++)
-#pragma unroll
-                for (int i = 0; i < 4; i++)
-#pragma unroll
-                    for (int j = 0; j < 4; j++) blk[mat][i][j] = 0.f;
-            // CPU order inside a block: Q8_0 k = 0..31; Q4_0 k = j, j+16 for j = 0..15.
-#pragma unroll 4
-            for (int s = 0; s < FK; s++) {
-                const int k = FMT == DT_Q4_0 ? ((s & 1) ? 16 + (s >> 1) : (s >> 1)) : s;
-                const float4 xv = *(const float4*)&Xs[k][ty * 4];
-                const float xa[4] = {xv.x, xv.y, xv.z, xv.w};
-#pragma unroll
-                for (int mat = 0; mat < NB; mat++) {
-                    const float4 wv = *(const float4*)&Ws[mat][k][tx * 4];
-                    const float wa[4] = {wv.x, wv.y, wv.z, wv.w};
-#pragma unroll
-                    for (int i = 0; i < 4; i++)
-#pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            const float t = wa[j] * xa[i];
-                            blk[mat][i][j] += t;
-                        }
-                }
-            }
-#pragma unroll
-            for (int mat = 0; mat < NB; mat++)
-#pragma unroll
-                for (int j = 0; j < 4; j++) {
-                    const float d = Ds[mat][tx * 4 + j];
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const float t = d * blk[mat][i][j];
-                        acc[mat][i][j] += t;
-                    }
-                }
-        } else {
-#pragma unroll 4
-            for (int k = 0; k < FK; k++) {
-                const float4 xv = *(const float4*)&Xs[k][ty * 4];
-                const float xa[4] = {xv.x, xv.y, xv.z, xv.w};
-#pragma unroll
-                for (int mat = 0; mat < NB; mat++) {
-                    const float4 wv = *(const float4*)&Ws[mat][k][tx * 4];
-                    const float wa[4] = {wv.x, wv.y, wv.z, wv.w};
-#pragma unroll
-                    for (int i = 0; i < 4; i++)
-#pragma unroll
-                        for (int j = 0; j < 4; j++) {
-                            const float t = wa[j] * xa[i];
-                            acc[mat][i][j] += t;
-                        }
-                }
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const int m = m0 + ty * 4 + i;
-        if (m >= M) continue;
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const int n = n0 + tx * 4 + j;
-            if (n >= N) continue;
-            const int64_t o = (int64_t)m * p.ldy + n;
-            if (MODE == GEMM_STORE) {
-                p.y[o] = acc[0][i][j];
-            } else if (MODE == GEMM_ACC) {
-                p.y[o] = p.y[o] + acc[0][i][j];
+            const int64_t blk = (int64_t)n * nb + min(b, nb - 1);
+            if (FMT == DT_Q8_0) {
+                raw[mat][0] = gload_i4(w.q + blk * 32);
+                raw[mat][1] = gload_i4(w.q + blk * 32 + 16);
             } else {
-                const float g = acc[0][i][j];
-                const float e = expf(-g);
-                const float den = 1.0f + e;
-                p.y[o] = (g / den) * acc[NB - 1][i][j];
+                raw[mat][0] = gload_i4(w.q + blk * 16);
+            }
+            d[mat] = (float)*gptr(w.s + blk);
+        }
+    };
+    load(wave);
+    for (int ph = 0; ph < phases; ph++) {
+        const int b = ph * NW + wave;
+        float* buf = parts + (size_t)(ph & 1) * NW * NB * MT * 64;
+        if (b < nb) {
+            float blk[NB][MT];
+#pragma unroll
+            for (int mat = 0; mat < NB; mat++)
+#pragma unroll
+                for (int i = 0; i < MT; i++) blk[mat][i] = 0.f;
+            // CPU order inside a block: Q8_0 k = 0..31; Q4_0 k = j, j+16 for j = 0..15.
+#pragma unroll
+            for (int c = 0; c < 4; c++) {
+                float xs[MT][8];  // scalar registers
+#pragma unroll
+                for (int i = 0; i < MT; i++)
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+                        xs[i][e] = FMT == DT_Q8_0 ? xr[i][32 * b + 8 * c + e]
+                                                  : xr[i][32 * b + (e & 1) * 16 + 4 * c + (e >> 1)];
+#pragma unroll
+                for (int mat = 0; mat < NB; mat++) {
+                    float wv[8];
+                    if (FMT == DT_Q8_0) {
+                        const int4 q = raw[mat][c >> 1];
+                        const uint32_t u0 = (uint32_t)((c & 1) ? q.z : q.x) ^ 0x80808080u;
+                        const uint32_t u1 = (uint32_t)((c & 1) ? q.w : q.y) ^ 0x80808080u;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {  // q + 128, exactly, then q
+                            wv[e] = (float)((u0 >> (8 * e)) & 255u) - 128.0f;
+                            wv[4 + e] = (float)((u1 >> (8 * e)) & 255u) - 128.0f;
+                        }
+                    } else {
+                        const int4 q = raw[mat][0];
+                        const uint32_t u = (uint32_t)(c == 0 ? q.x : c == 1 ? q.y : c == 2 ? q.z : q.w);
+                        const uint32_t lo = u & 0x0F0F0F0Fu, hi = (u >> 4) & 0x0F0F0F0Fu;
+#pragma unroll
+                        for (int e = 0; e < 4; e++) {
+                            wv[2 * e] = (float)((lo >> (8 * e)) & 255u) - 8.0f;
+                            wv[2 * e + 1] = (float)((hi >> (8 * e)) & 255u) - 8.0f;
+                        }
+                    }
+#pragma unroll
+                    for (int e = 0; e < 8; e++)
+#pragma unroll
+                        for (int i = 0; i < MT; i++) {
+                            const float t = wv[e] * xs[i][e];
+                            blk[mat][i] += t;
+                        }
+                }
+            }
+#pragma unroll
+            for (int mat = 0; mat < NB; mat++)
+#pragma unroll
+                for (int i = 0; i < MT; i++) buf[((wave * NB + mat) * MT + i) * 64 + lane] = d[mat] * blk[mat][i];
+        }
+        if (ph + 1 < phases) load(b + NW);
+        // (a buffer is written again two phases later, past the barrier that
+        // follows its reads: one barrier a phase is enough)
+        __syncthreads();
+        const int cnt = min(NW, nb - ph * NW);
+#pragma unroll
+        for (int k = 0; k < kOwn; k++) {
+            const int i = wave + k * NW;
+            if (i >= MT) break;
+#pragma unroll
+            for (int mat = 0; mat < NB; mat++)
+                for (int v = 0; v < cnt; v++) acc[mat][k] += buf[((v * NB + mat) * MT + i) * 64 + lane];
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < kOwn; k++) {
+        const int i = wave + k * NW;
+        if (i >= MT) break;
+        if (m0 + i < M && n0 + lane < N) f32_finish<MODE>(p, m0 + i, n0 + lane, acc[0][k], acc[NB - 1][k]);
+    }
+}
+
+// F16 weights have no blocks: each output is one chain over K.  A lane owns a
+// weight row, a wave MT rows of activations, a workgroup 4 waves.
+template <int MODE, int MT>
+__global__ __launch_bounds__(256) void gemm_f32_half_kernel(GemmF32Args p) {
+#pragma clang fp contract(off)
+    constexpr int NB = MODE == GEMM_SWIGLU ? 2 : 1;
+    const int K = p.w.cols, N = p.w.rows, M = p.M, lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = blockIdx.y * 64, m0 = (blockIdx.x * 4 + wave) * MT, n = min(n0 + lane, N - 1);
+    if (m0 >= M) return;
+    scalar_f32 xr[MT];
+#pragma unroll
+    for (int i = 0; i < MT; i++) xr[i] = (scalar_f32)(p.x + (int64_t)min(m0 + i, M - 1) * p.ldx);
+    float acc[NB][MT];
+#pragma unroll
+    for (int mat = 0; mat < NB; mat++)
+#pragma unroll
+        for (int i = 0; i < MT; i++) acc[mat][i] = 0.f;
+    constexpr int D = 4;  // 8-weight chunks in flight (K is a multiple of 32)
+    int4 raw[D][NB], nxt[D][NB];
+    auto load = [&](int k, int4 (&r)[D][NB]) {
+#pragma unroll
+        for (int s = 0; s < D; s++)
+#pragma unroll
+            for (int mat = 0; mat < NB; mat++)
+                r[s][mat] = gload_i4((mat ? p.u : p.w).q + ((int64_t)n * K + k + 8 * s) * 2);
+    };
+    load(0, nxt);
+    for (int k0 = 0; k0 < K; k0 += 8 * D) {
+#pragma unroll
+        for (int s = 0; s < D; s++)
+#pragma unroll
+            for (int mat = 0; mat < NB; mat++) raw[s][mat] = nxt[s][mat];
+        load(min(k0 + 8 * D, K - 8 * D), nxt);
+#pragma unroll
+        for (int s = 0; s < D; s++) {
+            float xs[MT][8];
+#pragma unroll
+            for (int i = 0; i < MT; i++)
+#pragma unroll
+                for (int e = 0; e < 8; e++) xs[i][e] = xr[i][k0 + 8 * s + e];
+#pragma unroll
+            for (int mat = 0; mat < NB; mat++) {
+                const f16x8 h = __builtin_bit_cast(f16x8, raw[s][mat]);
+#pragma unroll
+                for (int e = 0; e < 8; e++)
+#pragma unroll
+                    for (int i = 0; i < MT; i++) {
+                        const float t = (float)h[e] * xs[i][e];
+                        acc[mat][i] += t;
+                    }
             }
         }
     }
+#pragma unroll
+    for (int i = 0; i < MT; i++)
+        if (m0 + i < M && n0 + lane < N) f32_finish<MODE>(p, m0 + i, n0 + lane, acc[0][i], acc[NB - 1][i]);
+}
+
+// Waves per workgroup: the blocks of a row in even phases of at most 16.
+int f32_waves(int nb) {
+    const int phases = (nb + 15) / 16;
+    return (nb + phases - 1) / phases;
+}
+
+template <int FMT, int MODE, int MT>
+hipError_t run_f32_rows(const GemmF32Args& a, hipStream_t st) {
+    const int cols = (a.w.rows + 63) / 64;
+    if constexpr (FMT == DT_F16) {
+        gemm_f32_half_kernel<MODE, MT><<<dim3((a.M + 4 * MT - 1) / (4 * MT), cols), 256, 0, st>>>(a);
+    } else {
+        const int nw = f32_waves(a.w.cols / 32);
+        const size_t lds = (size_t)2 * nw * (MODE == GEMM_SWIGLU ? 2 : 1) * MT * 64 * 4;
+        auto* kernel = gemm_f32_kernel<FMT, MODE, MT>;
+        static const hipError_t attr =
+            hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10);
+        if (attr != hipSuccess) return attr;
+        kernel<<<dim3((a.M + MT - 1) / MT, cols), 64 * nw, lds, st>>>(a);
+    }
+    return hipGetLastError();
+}
+
+int device_cus();
+
+// Rows of activations per weight row a lane holds: as many as leave a workgroup
+// for every CU, since a lane's quants are converted once for all of them, and
+// at most four: eight rows' activations do not fit the scalar registers (gate+up
+// of the 135M shape over 150 rows: 90 us with eight, 38 with four; QKV 46 and
+// 12).  Against 64x64 tiles that walked K on one thread per 16 outputs, us: gate+up
+// 150 -> 38, QKV 85 -> 12, Wo and down 157 -> 15 (mean), Q8_0, 150 rows.
+template <int FMT, int MODE>
+hipError_t run_f32_mode(const GemmF32Args& a, hipStream_t st) {
+    const int64_t cols = (a.w.rows + 63) / 64, cus = device_cus();
+    const int per = FMT == DT_F16 ? 4 : 1;  // waves of a workgroup that take rows of their own
+    auto grid = [&](int mt) { return cols * ((a.M + per * mt - 1) / (per * mt)); };
+    if (grid(4) >= cus) return run_f32_rows<FMT, MODE, 4>(a, st);
+    if (grid(2) >= cus) return run_f32_rows<FMT, MODE, 2>(a, st);
+    return run_f32_rows<FMT, MODE, 1>(a, st);
 }
 
 template <int FMT>
 hipError_t run_f32(const GemmF32Args& a, int mode, hipStream_t st) {
-    dim3 grid((a.M + FB - 1) / FB, (a.w.rows + FB - 1) / FB);
-    if (mode == GEMM_STORE) gemm_f32_kernel<FMT, GEMM_STORE><<<grid, 256, 0, st>>>(a);
-    else if (mode == GEMM_ACC) gemm_f32_kernel<FMT, GEMM_ACC><<<grid, 256, 0, st>>>(a);
-    else gemm_f32_kernel<FMT, GEMM_SWIGLU><<<grid, 256, 0, st>>>(a);
-    return hipGetLastError();
+    if (mode == GEMM_STORE) return run_f32_mode<FMT, GEMM_STORE>(a, st);
+    if (mode == GEMM_ACC) return run_f32_mode<FMT, GEMM_ACC>(a, st);
+    return run_f32_mode<FMT, GEMM_SWIGLU>(a, st);
 }
 
 }  // namespace
