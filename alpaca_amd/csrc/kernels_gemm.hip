@@ -1315,6 +1315,23 @@ hipError_t pick_dgemm(const GemmArgs& a, hipStream_t st) {
     auto small_grid = [&](double per_cu) {
         return f == 0 && TT && tiles(128, 64) <= per_cu * cus;
     };
+    // One term, small grids (at most 1.6 tiles of 128x64 per CU): 64x64 tiles as
+    // well, and two K sets where those are at most one per CU (two at K >= 2,048;
+    // not for SwiGLU past one).  us a launch, 128x64 -> 64x64 / two sets: 135M
+    // shape over 512 rows gate+up 13.8 -> 10.3 / 10.1, over 700 QKV 11.0 -> 8.6 /
+    // 7.7, over 2,048 gate+up 19.5 -> 17.5; 360M shape over 1,024 down 25.0 ->
+    // 20.5, over 512 QKV 14.2 -> 11.4 / 9.7; 1.7B shape over 300 down 72.6 -> 58.0
+    // / 39.2.  Two sets change the order of K, so only below 768 rows, the
+    // shortest half of a prompt split over two streams (one-term rows of a split
+    // and an unsplit prompt agree).
+    if constexpr (!TT && !TAIL) {
+        if (f == 0 && tiles(128, 64) <= 1.6 * cus) {
+            const int per_cu = MODE != GEMM_SWIGLU && a.w.cols >= 2048 ? 2 : 1;
+            if (M < 768 && tiles(64, 64) <= per_cu * cus)
+                return run_dgemm<FMT, 64, 64, 32, 32, MODE, RH, TT, 2, TAIL>(a, st);
+            return run_dgemm<FMT, 64, 64, 32, 32, MODE, RH, TT, 1, TAIL>(a, st);
+        }
+    }
     if constexpr (MODE == GEMM_SWIGLU) {
         if constexpr (!TT)
             if (f == 1) return run_dgemm<FMT, 256, 64, 128, 32, MODE, RH, TT, 1, TAIL>(a, st);
@@ -1347,6 +1364,14 @@ hipError_t pick_dgemm(const GemmArgs& a, hipStream_t st) {
                 const int t64 = tiles(128, 64), rem = t64 % slots;
                 const double c64 = t64 / slots + (rem ? (rem <= cus ? 0.6 : 1.0) : 0.0);
                 const double cw = ((tiles(128, 256) + cus - 1) / cus) * (a.w.cols >= 1536 ? 1.87 : 1.32);
+                // Long K (the 1.7B shape): 64x64 tiles, three per CU, cost 0.78 a
+                // round and leave less of the last one idle: QKV over 700 rows 69 ->
+                // 50 us, over 1,024 70 -> 64.
+                if (a.w.cols >= 1536) {
+                    const int t = tiles(64, 64), r = t % (3 * cus);
+                    const double cs = 0.78 * (t / (3 * cus) + (!r ? 0.0 : r <= cus ? 0.5 : r <= 2 * cus ? 0.75 : 1.0));
+                    if (cs < c64 && cs < cw) return run_dgemm<FMT, 64, 64, 32, 32, MODE, RH, TT, 1, TAIL>(a, st);
+                }
                 if (cw < c64) return run_dgemm<FMT, 128, 256, 64, 64, MODE, RH, TT, 1, TAIL>(a, st);
                 return run_dgemm<FMT, 128, 64, 64, 32, MODE, RH, TT, 1, TAIL>(a, st);
             }

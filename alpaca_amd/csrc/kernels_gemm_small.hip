@@ -404,7 +404,7 @@ hipError_t run_small(const SmallArgs& a, hipStream_t st) {
 }
 
 // Tile families, smallest first.  F16 weight stages are twice the size, and
-// SwiGLU keeps two of them: the largest family then has one stage in flight.
+// SwiGLU keeps two of them: the largest tile's then leave room for four waves.
 template <int FMT, int MODE, int NV>
 hipError_t run_family(int family, const SmallArgs& a, hipStream_t st) {
     constexpr int DW = FMT == DT_F16 && MODE == GEMM_SWIGLU ? 1 : 2;
@@ -415,7 +415,7 @@ hipError_t run_family(int family, const SmallArgs& a, hipStream_t st) {
         if constexpr (NV == 0) return run_small<FMT, MODE, 2, 2, 8, 1, 0>(a, st);
         break;
     case 3:
-        if constexpr (NV == 0) return run_small<FMT, MODE, 2, 4, 4, DW, 0>(a, st);
+        if constexpr (NV == 0) return run_small<FMT, MODE, 2, 4, DW == 1 ? 4 : 8, 1, 0>(a, st);
         break;
     }
     return hipErrorNotSupported;
@@ -462,12 +462,12 @@ int device_cus() {
 //   135M shape     QKV          gate+up       down         Wo
 //    11 rows    7.8 -> 3.6   10.0 -> 3.7   11.7 -> 3.9   6.7 -> 3.3
 //    64 rows    8.3 -> 3.8   10.8 -> 4.5   11.6 -> 4.0   6.5 -> 3.3
-//   256 rows    8.5 -> 4.9   11.2 -> 9.0   11.8 -> 6.0   6.5 -> 4.5
-//   512 rows    8.6 -> 7.2   11.5 (13.7)   11.9 -> 9.3   6.7 -> 6.2
+//   256 rows    8.5 -> 5.1   11.2 -> 7.9   11.8 -> 6.0   6.5 -> 4.5
+//   512 rows    8.6 -> 6.1   11.4 (13.9)   12.2 -> 7.7   6.8 -> 5.3
 //   1.7B shape
 //    11 rows   16.5 -> 6.2   28.8 -> 10.0  49.4 -> 9.3  15.0 -> 4.2
 //    64 rows   16.9 -> 12.4  29.0 -> 18.5  50.0 -> 13.4 14.8 -> 5.5
-//   256 rows   26.7 (31.4)   47.9 (54.9)   51.3 -> 31.6 15.2 -> 10.8
+//   300 rows   26.9 (31.4)   56.9 (61.6)   51.3 (47.2)  15.5 (15.2)
 // (figures in brackets: these tiles past one workgroup per CU, not taken).
 // With the RMSNorm in the kernel (the two smallest tiles, K <= 1,024), norm
 // kernel + GEMM -> one launch: 135M QKV at 64 rows 2.6 + 3.8 -> 5.2 us, gate+up
