@@ -785,10 +785,32 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* q, int ldq, 
         l = l * alpha + xor32_combine(xor16_combine(ps, AddOp()), AddOp());
 #pragma unroll
         for (int d = 0; d < DT; d++) o[d] *= alpha;
+        // A key that a query does not see has p = 0, which a matrix product makes
+        // NaN of where the key's value is an infinity or NaN: such a tile on the
+        // diagonal is summed key by key, for the queries that see the key.
+        bool odd = false;
+        if (k0 + 15 > start + t0)
 #pragma unroll
-        for (int r = 0; r < 4; r++)
+            for (int r = 0; r < 4; r++)
 #pragma unroll
-            for (int d = 0; d < DT; d++) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[r][d], p[r], o[d], 0, 0, 0);
+                for (int d = 0; d < DT; d++) odd |= !(fabsf(vv[r][d]) < INFINITY);
+        if (__builtin_amdgcn_ballot_w64(odd)) {
+            for (int kg = 0; kg < 4; kg++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int key = k0 + 4 * kg + r;
+                    const float pk = __shfl(p[r], 16 * kg + c16, 64);
+                    if (key > pos) continue;
+                    const KV* vr = vb + (int64_t)key * HD + 4 * g;
+#pragma unroll
+                    for (int d = 0; d < DT; d++) o[d] += pk * load4(vr + 16 * d);
+                }
+        } else {
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+#pragma unroll
+                for (int d = 0; d < DT; d++) o[d] = __builtin_amdgcn_mfma_f32_16x16x4f32(vv[r][d], p[r], o[d], 0, 0, 0);
+        }
         m = mn;
     }
     // o[d][r] = O(query c16, dim 16 d + 4 g + r)

@@ -41,3 +41,15 @@ def test_float32_attention_of_several_queries(hip_ops, tokens, start, heads, kv,
     assert_close(hip_ops.attention(q, k, v, start, "f32"), orc.attention(q, k, v, start), 2e-6, 1e-5, "f32 cache")
     assert_close(hip_ops.attention(q, k, v, start, "f16"), orc.attention(q, _f16(k), _f16(v), start), 2e-5, 1e-4,
                  "f16 cache")
+
+
+@pytest.mark.parametrize("tokens,start,hd", [(20, 0, 64), (16, 37, 32), (37, 5, 128)])
+def test_float32_attention_keeps_later_values_from_earlier_queries(hip_ops, tokens, start, hd):
+    """A value that is an infinity or NaN reaches the queries that see its key and no others."""
+    cap = start + tokens
+    q, k, v = rand((tokens, 4, hd), 811), rand((cap, 2, hd), 812), rand((cap, 2, hd), 813)
+    v[start + 9, 0, 3], v[start + tokens - 2, 1, hd - 1] = np.inf, np.nan
+    got, want = hip_ops.attention(q, k, v, start, "f32"), orc.attention(q, k, v, start)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    seen = np.isfinite(want)
+    assert_close(got[seen], want[seen], 2e-6, 1e-5, "finite outputs")
