@@ -233,6 +233,11 @@ hipError_t launch_dequant_f16(const DevMatrix& m, f16* out, hipStream_t st);
 size_t sample_scratch_bytes(int n);
 hipError_t launch_sample(const float* logits, int n, float temperature, int top_k, float top_p, double u,
                          int32_t* out, int* status, uint32_t* cand_idx, double* cand_p, hipStream_t st);
+// A call's inputs and logits between the device and pinned host memory
+// (`host`: its device address; 16-byte aligned for the logits).
+hipError_t launch_fetch_words(const int32_t* host, int32_t* out, int n, hipStream_t st);
+hipError_t launch_set_step(int32_t* token_out, int32_t token, int* pos_out, int pos, hipStream_t st);
+hipError_t launch_store_host(const float* x, float* host, int n, hipStream_t st);
 hipError_t launch_argmax(const float* logits, int n, int32_t* chain_token, int32_t* emitted, int slot,
                          int* pos_dev, hipStream_t st);
 // RoPE with a host-built (cos, sin) table [positions][hd/2]; q rotated in

@@ -683,6 +683,7 @@ struct ahip_session {
     std::vector<std::unique_ptr<DevBuf>> kc, vc;
     DevBuf x, xn, xh, qkv, qh, ctx, ctxh, ffn, ffnh, partials, logits, tokens, chain, dpos;
     float* logits_host = nullptr;
+    float* logits_mapped = nullptr;     // device address of logits_host
     int32_t* emitted_host = nullptr;   // pinned, mapped: the arg-max kernel writes tokens here
     int32_t* emitted_mapped = nullptr; // device address of emitted_host
     bool dec_split = false;            // split-K decode attention (else the generic kernel)
@@ -704,6 +705,7 @@ struct ahip_session {
     std::vector<unsigned long long> pdec_trace_host;
     std::map<std::string, std::pair<double, int>> pdec_stages;
     int32_t* tokens_host = nullptr;
+    int32_t* tokens_mapped = nullptr;  // device address of tokens_host
     int length = 0;
     std::atomic<int> busy{0};
     double last_gpu = 0, last_encode = 0;
@@ -1197,11 +1199,13 @@ extern "C" int ahip_session_create(ahip_model* m, int capacity, int max_batch, i
                 A{&s->partials, z.partials * 4}, A{&s->logits, z.logits * 4}, A{&s->tokens, (int64_t)capacity * 4},
                 A{&s->chain, 64}, A{&s->dpos, 64}})
         if (int rc = a.b->alloc(a.n)) return rc;
-    if (hipHostMalloc((void**)&s->logits_host, (size_t)c.vocab_size * 4, hipHostMallocDefault) != hipSuccess ||
+    if (hipHostMalloc((void**)&s->logits_host, (size_t)c.vocab_size * 4, hipHostMallocMapped) != hipSuccess ||
         hipHostMalloc((void**)&s->emitted_host, ((size_t)capacity + 8) * 4, hipHostMallocMapped) != hipSuccess ||
-        hipHostMalloc((void**)&s->tokens_host, ((size_t)capacity + 8) * 4, hipHostMallocDefault) != hipSuccess)
+        hipHostMalloc((void**)&s->tokens_host, ((size_t)capacity + 8) * 4, hipHostMallocMapped) != hipSuccess)
         return fail(AHIP_ERR_ALLOC, "pinned host allocation failed");
     HIP_OR(hipHostGetDevicePointer((void**)&s->emitted_mapped, s->emitted_host, 0), "hipHostGetDevicePointer");
+    HIP_OR(hipHostGetDevicePointer((void**)&s->logits_mapped, s->logits_host, 0), "hipHostGetDevicePointer");
+    HIP_OR(hipHostGetDevicePointer((void**)&s->tokens_mapped, s->tokens_host, 0), "hipHostGetDevicePointer");
     s->dec_split = attention_decode_supported(c.head_count, c.kv_head_count, c.head_dim) &&
                    attention_decode_session_split_len(capacity, c.head_count, c.kv_head_count) > 0;
     if (s->dec_split) {
@@ -1697,16 +1701,17 @@ extern "C" int ahip_session_forward(ahip_session* s, const int32_t* tokens, int 
     const bool persistent = n == 1 && s->pdec;
     if (persistent) {
         // one persistent launch: token in `chain`, position in `dpos`
-        s->tokens_host[1] = s->length;
-        HIP_OR(hipMemcpyAsync(s->chain.p, s->tokens_host, 4, hipMemcpyHostToDevice, s->stream), "token upload");
-        HIP_OR(hipMemcpyAsync(s->dpos.p, s->tokens_host + 1, 4, hipMemcpyHostToDevice, s->stream), "position upload");
+        HIP_OR(launch_set_step(s->chain.as<int32_t>(), tokens[0], s->dpos.as<int>(), s->length, s->stream),
+               "token upload");
         if (int rc = pdec_launch(s, true, false)) {
             hipStreamSynchronize(s->stream);
             return rc;
         }
     } else {
-        HIP_OR(hipMemcpyAsync(s->tokens.p, s->tokens_host, (size_t)n * 4, hipMemcpyHostToDevice, s->stream),
-               "token upload");
+        if (n == 1)
+            HIP_OR(launch_set_step(s->tokens.as<int32_t>(), tokens[0], nullptr, 0, s->stream), "token upload");
+        else
+            HIP_OR(launch_fetch_words(s->tokens_mapped, s->tokens.as<int32_t>(), n, s->stream), "token upload");
         for (int c0 = 0; c0 < n; c0 += s->max_batch) {
             const int cn = std::min(s->max_batch, n - c0);
             if (int rc = encode_chunk(s, s->tokens.as<int32_t>() + c0, cn, s->length + c0, c0 + cn == n)) {
@@ -1716,8 +1721,7 @@ extern "C" int ahip_session_forward(ahip_session* s, const int32_t* tokens, int 
         }
     }
     s->stage_end();
-    HIP_OR(hipMemcpyAsync(s->logits_host, s->logits.p, (size_t)s->m->c.vocab_size * 4, hipMemcpyDeviceToHost, s->stream),
-           "logits download");
+    HIP_OR(launch_store_host(s->logits.as<float>(), s->logits_mapped, s->m->c.vocab_size, s->stream), "logits download");
     HIP_OR(hipEventRecord(s->ev_end, s->stream), "hipEventRecord");
     s->last_encode = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     HIP_OR(hipStreamSynchronize(s->stream), "forward");
@@ -1805,10 +1809,7 @@ extern "C" int ahip_session_decode_greedy(ahip_session* s, int32_t start, int ma
     const bool use_pdec = s->pdec;
     const bool use_graph = !use_pdec && !s->profiling && capture_greedy_graph(s);
     s->begin_call();
-    s->tokens_host[0] = start;
-    s->tokens_host[1] = s->length;
-    HIP_OR(hipMemcpyAsync(s->chain.p, s->tokens_host, 4, hipMemcpyHostToDevice, st), "chain upload");
-    HIP_OR(hipMemcpyAsync(s->dpos.p, s->tokens_host + 1, 4, hipMemcpyHostToDevice, st), "position upload");
+    HIP_OR(launch_set_step(s->chain.as<int32_t>(), start, s->dpos.as<int>(), s->length, st), "chain upload");
     HIP_OR(hipEventRecord(s->ev_begin, st), "hipEventRecord");
     std::vector<hipEvent_t> done(budget, nullptr);
     int submitted = 0, fed = 0, rc = AHIP_OK;
