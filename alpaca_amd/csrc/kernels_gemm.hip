@@ -25,7 +25,8 @@
 // Epilogues: store f32, accumulate into the f32 residual, or SwiGLU
 // (silu(x Wg^T) * (x Wu^T) from two accumulator sets) written as f16.
 //
-// gemm_f32_kernel (exact): float32 on the VALU.  Inside a block the products are
+// gemm_f32_kernel, gemm_f32_half_kernel, gemm_f32_tile_kernel (exact; few rows,
+// few rows of F16 weights, full grids): float32 on the VALU.  Inside a block the products are
 // summed in the CPU reference's order and the block sum is scaled once
 // (acc += d * s), with FP contraction off, so each output equals the CPU
 // reference's float32 result.
@@ -337,9 +338,10 @@ __device__ __forceinline__ void f32_finish(const GemmF32Args& p, int m, int n, f
 // independent of each other: a workgroup's waves take one block each, and the
 // scaled sums meet in LDS, where one thread per output adds them in order (the
 // same bits as one thread walking K).  A lane owns a weight row (64 per wave),
-// so a block's quants are converted once for MT rows of activations, which are
-// wave-uniform and come as scalar operands: two VALU instructions per product
-// and nothing else, the least that separate roundings of product and sum allow.
+// so a block's quants are converted (a conversion and a subtraction each) once for
+// MT rows of activations, which are wave-uniform and come as scalar operands, so a
+// product costs a multiplication and an addition, the least that their separate
+// roundings allow: 2.5 VALU instructions a product at MT = 4, 4 at MT = 1.
 template <int FMT, int MODE, int MT>
 __global__ __launch_bounds__(1024) void gemm_f32_kernel(GemmF32Args p) {
 #pragma clang fp contract(off)
@@ -516,6 +518,120 @@ __global__ __launch_bounds__(256) void gemm_f32_half_kernel(GemmF32Args p) {
         if (m0 + i < M && n0 + lane < N) f32_finish<MODE>(p, m0 + i, n0 + lane, acc[0][i], acc[NB - 1][i]);
 }
 
+// Full grids: 64x64 tiles, 4x4 outputs a thread over LDS tiles of one quant block
+// of K, the same order of sums.  A weight is unpacked once for 64 rows, which is
+// what counts where every CU has workgroups enough to hide the stages' round trips.
+constexpr int FB = 64;      // tile edge (tokens and rows)
+constexpr int FK = 32;      // one quant block per stage
+constexpr int FP = FB + 4;  // LDS pitch in floats
+
+// Weight (row n, column k) as an unscaled value: q for Q8_0, nib-8 for Q4_0,
+// the f16 value for F16.  The block scale is applied once per block sum.
+template <int FMT>
+__device__ __forceinline__ float w_raw(const DevMatrix& m, int n, int k, int K) {
+    if (FMT == DT_Q8_0) return (float)((const int8_t*)m.q)[(int64_t)n * K + k];
+    if (FMT == DT_Q4_0) {
+        const int j = k & 31;
+        const uint8_t b = m.q[((int64_t)n * (K >> 5) + (k >> 5)) * 16 + (j & 15)];
+        return (float)((int)(j < 16 ? (b & 15) : (b >> 4)) - 8);
+    }
+    return (float)((const f16*)m.q)[(int64_t)n * K + k];
+}
+
+template <int FMT, int MODE>
+__global__ __launch_bounds__(256) void gemm_f32_tile_kernel(GemmF32Args p) {
+#pragma clang fp contract(off)
+    constexpr int NB = MODE == GEMM_SWIGLU ? 2 : 1;
+    constexpr bool kQuant = FMT != DT_F16;
+    __shared__ float Xs[FK][FP];
+    __shared__ float Ws[NB][FK][FP];
+    __shared__ float Ds[NB][FB];
+
+    const int K = p.w.cols, N = p.w.rows, M = p.M;
+    const int m0 = blockIdx.x * FB, n0 = blockIdx.y * FB;
+    const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
+
+    float acc[NB][4][4];
+#pragma unroll
+    for (int mat = 0; mat < NB; mat++)
+#pragma unroll
+        for (int i = 0; i < 4; i++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) acc[mat][i][j] = 0.f;
+
+    const int lr = tid >> 2, lk = (tid & 3) * 8;
+    for (int k0 = 0; k0 < K; k0 += FK) {
+        {
+            const int m = m0 + lr;
+#pragma unroll
+            for (int j = 0; j < 8; j++) Xs[lk + j][lr] = m < M ? p.x[(int64_t)m * p.ldx + k0 + lk + j] : 0.f;
+        }
+#pragma unroll
+        for (int mat = 0; mat < NB; mat++) {
+            const DevMatrix& w = mat ? p.u : p.w;
+            const int n = n0 + lr;
+#pragma unroll
+            for (int j = 0; j < 8; j++) Ws[mat][lk + j][lr] = n < N ? w_raw<FMT>(w, n, k0 + lk + j, K) : 0.f;
+            if (kQuant && lk == 0) Ds[mat][lr] = n < N ? (float)w.s[(int64_t)n * (K >> 5) + (k0 >> 5)] : 0.f;
+        }
+        __syncthreads();
+        // A quant block's products sum to blk, which its scale adds to acc; F16
+        // weights have no blocks and sum in acc.
+        float blk[NB][4][4];
+#pragma unroll
+        for (int mat = 0; mat < NB; mat++)
+#pragma unroll
+            for (int i = 0; i < 4; i++)
+#pragma unroll
+                for (int j = 0; j < 4; j++) blk[mat][i][j] = kQuant ? 0.f : acc[mat][i][j];
+        // CPU order inside a block: Q8_0 k = 0..31; Q4_0 k = j, j+16 for j = 0..15.
+#pragma unroll 4
+        for (int s = 0; s < FK; s++) {
+            const int k = FMT == DT_Q4_0 ? ((s & 1) ? 16 + (s >> 1) : (s >> 1)) : s;
+            const float4 xv = *(const float4*)&Xs[k][ty * 4];
+            const float xa[4] = {xv.x, xv.y, xv.z, xv.w};
+#pragma unroll
+            for (int mat = 0; mat < NB; mat++) {
+                const float4 wv = *(const float4*)&Ws[mat][k][tx * 4];
+                const float wa[4] = {wv.x, wv.y, wv.z, wv.w};
+#pragma unroll
+                for (int i = 0; i < 4; i++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const float t = wa[j] * xa[i];
+                        blk[mat][i][j] += t;
+                    }
+            }
+        }
+#pragma unroll
+        for (int mat = 0; mat < NB; mat++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const float d = kQuant ? Ds[mat][tx * 4 + j] : 0.f;
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    if constexpr (kQuant) {
+                        const float t = d * blk[mat][i][j];
+                        acc[mat][i][j] += t;
+                    } else {
+                        acc[mat][i][j] = blk[mat][i][j];
+                    }
+                }
+            }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const int m = m0 + ty * 4 + i;
+        if (m >= M) continue;
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int n = n0 + tx * 4 + j;
+            if (n < N) f32_finish<MODE>(p, m, n, acc[0][i][j], acc[NB - 1][i][j]);
+        }
+    }
+}
+
 // Waves per workgroup: the blocks of a row in even phases of at most 16.
 int f32_waves(int nb) {
     const int phases = (nb + 15) / 16;
@@ -541,15 +657,33 @@ hipError_t run_f32_rows(const GemmF32Args& a, hipStream_t st) {
 
 int device_cus();
 
-// Rows of activations per weight row a lane holds: as many as leave a workgroup
-// for every CU, since a lane's quants are converted once for all of them, and
-// at most four: eight rows' activations do not fit the scalar registers (gate+up
-// of the 135M shape over 150 rows: 90 us with eight, 38 with four; QKV 46 and
-// 12).  Against 64x64 tiles that walked K on one thread per 16 outputs, us: gate+up
-// 150 -> 38, QKV 85 -> 12, Wo and down 157 -> 15 (mean), Q8_0, 150 rows.
+// The kernels against each other.  A 64x64 tile walks K on one thread per 16
+// outputs, 0.14-0.15 us a column of K (0.25 with SwiGLU's two matrices) however
+// few rows there are, and runs at 20-23 products a ns once it has covered the chip
+// about three times; the kernels above need no more than a workgroup per CU but
+// stop at 10-12 (Q8_0), 5 (Q4_0) and 13-18 (F16), since they unpack a weight once
+// for every four rows.  Both sides grow with K, so the line is a number of outputs
+// per CU, in 64x64 tiles: 1.5 (Q8_0), 0.62 (Q4_0), 2.2 (F16).  us a launch, block per wave / 64x64:
+//   Q8_0 135M shape gate+up   150 rows   39 / 150    512   97 / 145   1,024  185 / 150   4,096  669 / 338
+//             "     QKV       150 rows   13 /  86  1,024   55 /  84   2,048  104 /  85   4,096  199 / 131
+//             "     down      150 rows   21 / 225  1,024   83 / 218   2,048  159 / 217   4,096  325 / 283
+//   Q8_0 1.7B shape gate+up    64 rows  211 / 503    150  472 / 555     256  755 / 552   2,048 5,999 / 2,980
+//   Q4_0 360M shape gate+up   150 rows  167 / 249    256  272 / 248     512  533 / 255   2,048 2,091 / 514
+//   F16  135M shape gate+up   512 rows   66 / 147  2,048  235 / 211
+//   F16  1.7B shape gate+up   150 rows  366 / 542    512 1,034 / 822  2,048 3,672 / 2,643
+// Rows of activations per weight row a lane holds, below that line: as many as
+// leave a workgroup for every CU, since a lane's quants are converted once for all
+// of them, and at most four: eight rows' activations do not fit the scalar
+// registers (gate+up of the 135M shape over 150 rows: 90 us with eight, 38 with
+// four; QKV 46 and 12).
 template <int FMT, int MODE>
 hipError_t run_f32_mode(const GemmF32Args& a, hipStream_t st) {
     const int64_t cols = (a.w.rows + 63) / 64, cus = device_cus();
+    constexpr double kFull = FMT == DT_Q8_0 ? 1.5 : FMT == DT_Q4_0 ? 0.62 : 2.2;
+    if ((double)a.M * a.w.rows >= kFull * (FB * FB) * (double)cus) {
+        gemm_f32_tile_kernel<FMT, MODE><<<dim3((a.M + FB - 1) / FB, (int)cols), 256, 0, st>>>(a);
+        return hipGetLastError();
+    }
     const int per = FMT == DT_F16 ? 4 : 1;  // waves of a workgroup that take rows of their own
     auto grid = [&](int mt) { return cols * ((a.M + per * mt - 1) / (per * mt)); };
     if (grid(4) >= cus) return run_f32_rows<FMT, MODE, 4>(a, st);

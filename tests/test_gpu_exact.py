@@ -1,12 +1,13 @@
-"""The float32 kernels of the exact mode: the GEMM whose workgroups' waves take
-a 32-weight block each (bit for bit the CPU reference's sums) and the attention
-of several queries on the float32 matrix instructions.
+"""The float32 kernels of the exact mode: the GEMMs, whose workgroups' waves take
+a 32-weight block each or, on full grids, 64x64 tiles (bit for bit the CPU
+reference's sums), and the attention of several queries on the float32 matrix
+instructions.
 """
 import numpy as np
 import pytest
 
 import oracle.oracle as orc
-from alpaca_amd.tensor import encode
+from alpaca_amd.tensor import F16, Q4_0, Q8_0, encode
 from tests.helpers import assert_close
 from tests.test_gpu_kernels import FORMATS, _f16, rand
 
@@ -23,6 +24,20 @@ def test_exact_gemm_bits(hip_ops, name, dt, m, n, k):
     GEMM's tolerance (expf differs from the host's in the last bit)."""
     x, res = rand((m, k), 700 + m), rand((m, n), 701, 5)
     w, wu = encode(rand((n, k), 702, 0.3), dt), encode(rand((n, k), 703, 0.3), dt)
+    y, u = orc.linear(x, dt, w.data, n), orc.linear(x, dt, wu.data, n)
+    for what, got, want in (("store", hip_ops.linear(x, w, "exact"), y),
+                            ("residual", hip_ops.linear_add(x, w, res, "exact"), orc.add(res, y))):
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), f"{name} {what}"
+    assert_close(hip_ops.gate_up_silu(x, w, wu, "exact"), orc.mul(orc.silu(y), u), 2e-4, 1e-4, f"{name} swiglu")
+
+
+@pytest.mark.parametrize("name,dt,m,n,k", [("Q8_0", Q8_0, 1061, 1490, 96), ("Q4_0", Q4_0, 1061, 640, 544),
+                                           ("F16", F16, 1301, 1800, 64), ("Q8_0", Q8_0, 25000, 65, 32)])
+def test_exact_gemm_bits_on_full_grids(hip_ops, name, dt, m, n, k):
+    """Outputs past the 64x64 tiles' share of a 256-CU chip (1.5, 0.62 and 2.2 tiles a CU), partial
+    tiles in both directions: bit for bit as in test_exact_gemm_bits."""
+    x, res = rand((m, k), 720, 1), rand((m, n), 721, 5)
+    w, wu = encode(rand((n, k), 722, 0.3), dt), encode(rand((n, k), 723, 0.3), dt)
     y, u = orc.linear(x, dt, w.data, n), orc.linear(x, dt, wu.data, n)
     for what, got, want in (("store", hip_ops.linear(x, w, "exact"), y),
                             ("residual", hip_ops.linear_add(x, w, res, "exact"), orc.add(res, y))):
