@@ -1384,6 +1384,8 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
     // a call's activations keep float32 grade whatever the session's precision
     // (one MFMA tile of rows costs the same with one term or two).
     const bool few = n < 16;
+    // ... and its weights: the quants, not the f16 copies of the prefill weight cache
+    auto pre = [&](const OwnedMatrix& w, const OwnedMatrix& h) -> const DevMatrix& { return few ? w.m : L.pre(w, h); };
     const int lo = few ? kLoAll : s->two_term ? s->lo_terms : 0;
     const bool all = s->lo_all_rows || few;
     const int tail0 = all ? 0 : last ? (n - 1) / 256 * 256 : n;
@@ -1407,7 +1409,7 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
         return in;
     };
     const int none = 1 << 30;  // a first row past the last: no second terms
-    const DevMatrix& wqkv = L.pre(L.qkv, L.qkv16);
+    const DevMatrix& wqkv = pre(L.qkv, L.qkv16);
     hipError_t fused = hipErrorNotSupported;
     const bool rope_fused = flash && s->fuse_qkv_rope;
     QkvRope o;
@@ -1490,7 +1492,7 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
     const int side = (!all && last && tail0 > 0) ? last_row_gemv_mask(L, n) : 0;
     const int64_t lr = n - 1;  // the last row
     s->stage("attn out projection (+residual)");
-    const DevMatrix& wo = L.pre(L.wo, L.wo16);
+    const DevMatrix& wo = pre(L.wo, L.wo16);
     if ((side & kSideWo) && ctxhlo) {
         LAUNCH(launch_gemm_mfma(ctxh, nullptr, QW, n - 1, wo, nullptr, x, nullptr, nullptr, H, GEMM_ACC, st));
         LAUNCH(launch_gemv_pair(wo, nullptr, ctxh + lr * QW, ctxhlo + lr * QW, x + lr * H, nullptr, nullptr, GEMV_ADD,
@@ -1498,7 +1500,7 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
     } else {
         LAUNCH(launch_gemm_mfma(ctxh, ctxhlo, QW, n, wo, nullptr, x, nullptr, nullptr, H, GEMM_ACC, st, lo_tile));
     }
-    const DevMatrix &wg = L.pre(L.gate, L.gate16), &wu = L.pre(L.up, L.up16);
+    const DevMatrix &wg = pre(L.gate, L.gate16), &wu = pre(L.up, L.up16);
     const bool side_gu = (side & kSideGateUp) && xhlo_ffn && ffnhlo;
     const SmallGemmInput ffn_in = normed_row(L.ffn_norm);
     const bool ffn_normed = !side_gu && gemm_small_takes(ffn_in, n, wg, &wu);
@@ -1518,7 +1520,7 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
         LAUNCH(launch_gemm_mfma(xh, xhlo_ffn, H, n, wg, &wu, nullptr, ffnh, ffnhlo, F, GEMM_SWIGLU, st, lo_tile, tail0));
     }
     s->stage("ffn down (+residual)");
-    const DevMatrix& wd = L.pre(L.down, L.down16);
+    const DevMatrix& wd = pre(L.down, L.down16);
     if ((side & kSideDown) && ffnhlo) {
         LAUNCH(launch_gemm_mfma(ffnh, nullptr, F, n - 1, wd, nullptr, x, nullptr, nullptr, H, GEMM_ACC, st));
         LAUNCH(launch_gemv_pair(wd, nullptr, ffnh + lr * F, ffnhlo + lr * F, x + lr * H, nullptr, nullptr, GEMV_ADD,
