@@ -713,22 +713,23 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(const float* q, int ld
     }
 }
 
-// Several queries in float32 (exact prefill, f32 cache, head dims the flash
-// kernel does not take): a workgroup takes 16 queries of one head, its four
-// waves every fourth tile of 16 keys, with online softmax states that merge in
-// LDS.  Products run on the float32 matrix instructions (f32 operands, f32
+// Several queries in float32 (exact prefill, f32 cache, calls of 2 to 15 tokens,
+// head dims the flash kernel does not take): a workgroup takes 16 queries of one
+// head, its NW waves every NW-th tile of 16 keys, with online softmax states that
+// merge in LDS.  Products run on the float32 matrix instructions (f32 operands, f32
 // sums): S^T = K Q^T leaves lane (g, c) with the scores of keys 4g..4g+3 for
 // query c, which is the B operand of O^T += V^T P^T when its four keys of step
 // r are taken as {4g + r}, so no probability crosses lanes.  K's dims are
 // paired with Q's in the same permuted order (16 B of a row per lane).  The
 // generic kernel below walks one query per wave, a key per lane and then a key
 // at a time: 150 queries of the 135M shape 55 us -> 8.6.
-template <int HD, typename KV>
-__global__ __launch_bounds__(256) void attn_f32_kernel(const float* q, int ldq, const KV* kc, const KV* vc, int cap,
-                                                       int H, int KVH, int T, int start, float* out, float scale) {
+template <int HD, typename KV, int NW>
+__global__ __launch_bounds__(64 * NW) void attn_f32_kernel(const float* q, int ldq, const KV* kc, const KV* vc,
+                                                           int cap, int H, int KVH, int T, int start, float* out,
+                                                           float scale) {
     constexpr int KC = HD / 16, DT = HD / 16;
-    __shared__ float xo[4][16][HD];  // partial outputs, [wave][query][dim]
-    __shared__ float xml[4][2][16];  // the waves' max and sum
+    __shared__ float xo[NW][16][HD];  // partial outputs, [wave][query][dim]
+    __shared__ float xml[NW][2][16];  // the waves' max and sum
     const int h = blockIdx.x, t0 = blockIdx.y * 16, kvh = h / (H / KVH);
     const int lane = threadIdx.x & 63, g = lane >> 4, c16 = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -751,7 +752,7 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* q, int ldq, 
 #pragma unroll
     for (int d = 0; d < DT; d++) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m = -INFINITY, l = 0.f;
-    for (int k0 = wave * 16; k0 < kend; k0 += 64) {
+    for (int k0 = wave * 16; k0 < kend; k0 += 16 * NW) {
         // rows past the last key repeat it (masked below)
         const KV* kr = kb + (int64_t)min(k0 + c16, kend - 1) * HD + 4 * g;
         f32x4 kv[KC];
@@ -821,15 +822,15 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* q, int ldq, 
         xml[wave][1][c16] = l;
     }
     __syncthreads();
-    for (int i = threadIdx.x; i < 16 * HD; i += 256) {
+    for (int i = threadIdx.x; i < 16 * HD; i += 64 * NW) {
         const int qr = i / HD, d = i % HD;
         if (t0 + qr >= T) break;
         float mt = xml[0][0][qr];  // finite: the first wave saw key 0
 #pragma unroll
-        for (int w = 1; w < 4; w++) mt = fmaxf(mt, xml[w][0][qr]);
+        for (int w = 1; w < NW; w++) mt = fmaxf(mt, xml[w][0][qr]);
         float lt = 0.f, ot = 0.f;
 #pragma unroll
-        for (int w = 0; w < 4; w++) {
+        for (int w = 0; w < NW; w++) {
             const float a = expf(xml[w][0][qr] - mt);
             lt += a * xml[w][1][qr];
             ot += a * xo[w][qr][d];
@@ -838,16 +839,34 @@ __global__ __launch_bounds__(256) void attn_f32_kernel(const float* q, int ldq, 
     }
 }
 
+template <int HD, typename KV>
+void run_attn_f32_hd(bool wide, dim3 grid, hipStream_t st, const float* q, int ldq, const KV* kc, const KV* vc, int cap,
+                     int H, int KVH, int T, int start, float* out, float scale) {
+    constexpr int kWide = HD <= 64 ? 16 : 8;  // (64 KB of partial outputs)
+    if (wide)
+        attn_f32_kernel<HD, KV, kWide><<<grid, 64 * kWide, 0, st>>>(q, ldq, kc, vc, cap, H, KVH, T, start, out, scale);
+    else
+        attn_f32_kernel<HD, KV, 4><<<grid, 256, 0, st>>>(q, ldq, kc, vc, cap, H, KVH, T, start, out, scale);
+}
+
+// Waves: four, whose states merge quickly, or where few queries leave most CUs idle
+// (at most 64 workgroups; calls of up to 15 tokens have one per head) and the keys
+// give four waves more than two tiles each, as many as fit.  11 queries of the 135M
+// shape, us, four waves / sixteen: 300 keys 14 / 8, 2,000 keys 66 / 28.
+constexpr int64_t kWideGrid = 64;
+constexpr int kWideKeys = 128;
 template <typename KV>
-bool run_attn_f32(int hd, dim3 grid, hipStream_t st, const float* q, int ldq, const void* kc, const void* vc, int cap,
-                  int H, int KVH, int T, int start, float* out, float scale) {
+bool run_attn_f32(int hd, hipStream_t st, const float* q, int ldq, const void* kc, const void* vc, int cap, int H,
+                  int KVH, int T, int start, float* out, float scale) {
+    const dim3 grid(H, (T + 15) / 16);
+    const bool wide = (int64_t)grid.x * grid.y <= kWideGrid && start + T > kWideKeys;
     const KV* k = (const KV*)kc;
     const KV* v = (const KV*)vc;
     switch (hd) {
-    case 32: attn_f32_kernel<32, KV><<<grid, 256, 0, st>>>(q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
-    case 64: attn_f32_kernel<64, KV><<<grid, 256, 0, st>>>(q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
-    case 96: attn_f32_kernel<96, KV><<<grid, 256, 0, st>>>(q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
-    case 128: attn_f32_kernel<128, KV><<<grid, 256, 0, st>>>(q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
+    case 32: run_attn_f32_hd<32, KV>(wide, grid, st, q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
+    case 64: run_attn_f32_hd<64, KV>(wide, grid, st, q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
+    case 96: run_attn_f32_hd<96, KV>(wide, grid, st, q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
+    case 128: run_attn_f32_hd<128, KV>(wide, grid, st, q, ldq, k, v, cap, H, KVH, T, start, out, scale); return true;
     default: return false;
     }
 }
@@ -1352,11 +1371,10 @@ hipError_t launch_attention_generic(const float* q, int ldq, const void* kc, con
     // several queries: tiles of 16 (rows of 16-byte alignment; head dims past 128
     // would hold too many accumulators)
     if (tokens > 1 && splits == 1 && !((uintptr_t)q & 15) && ldq % 4 == 0) {
-        const dim3 tiles(heads, (tokens + 15) / 16);
-        const bool took = kv_f16 ? run_attn_f32<f16>(hd, tiles, st, q, ldq, kc, vc, capacity, heads, kv_heads, tokens,
-                                                     start, out, scale)
-                                 : run_attn_f32<float>(hd, tiles, st, q, ldq, kc, vc, capacity, heads, kv_heads,
-                                                       tokens, start, out, scale);
+        const bool took = kv_f16 ? run_attn_f32<f16>(hd, st, q, ldq, kc, vc, capacity, heads, kv_heads, tokens, start,
+                                                     out, scale)
+                                 : run_attn_f32<float>(hd, st, q, ldq, kc, vc, capacity, heads, kv_heads, tokens,
+                                                       start, out, scale);
         if (took) return hipGetLastError();
     }
     dim3 grid(splits, heads, tokens);

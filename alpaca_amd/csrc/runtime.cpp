@@ -1620,7 +1620,9 @@ static int encode_chunk(ahip_session* s, const int32_t* dtok, int n, int pos, bo
     // (below 16 rows every operand takes its second term, encode_mfma_layer; without the flash
     // kernel those calls stay on the float32 kernels)
     const bool mfma = s->fast && !s->prefill_f32_gemm && (n >= 16 || flash_fits);
-    const bool flash = flash_fits && (n >= 16 || mfma);
+    // the flash kernel takes q and P as f16 terms and multiplies every value of a key block, also
+    // those of later keys, by p = 0: below 16 rows attention stays on the float32 kernel
+    const bool flash = flash_fits && n >= 16;
     if (mfma && n >= env_int("ALPACA_HIP_SPLIT_MIN", kSplitPrefillMin) && !s->profiling && env_int("ALPACA_HIP_PREFILL_STREAMS", 2) >= 2 &&
         prefill_split_pays(n, QW + 2 * KW)) {
         if (!s->part_stream[1]) s->part_stream[1] = split_stream_acquire(m->device);

@@ -58,6 +58,19 @@ def test_float32_attention_of_several_queries(hip_ops, tokens, start, heads, kv,
                  "f16 cache")
 
 
+@pytest.mark.parametrize("tokens,start,heads,kv,hd", [(2, 126, 9, 3, 64), (2, 127, 9, 3, 64), (11, 1013, 32, 32, 64),
+                                                      (15, 300, 4, 2, 32), (9, 2000, 8, 2, 128), (13, 131, 4, 4, 96),
+                                                      (20, 600, 32, 8, 64), (33, 600, 32, 8, 64)])
+def test_float32_attention_of_few_queries_over_many_keys(hip_ops, tokens, start, heads, kv, hd):
+    """Both sides of the rules for eight or sixteen waves a workgroup (128 keys, 64 workgroups): the
+    tolerances of test_float32_attention_of_several_queries."""
+    cap = start + tokens + 3
+    q, k, v = rand((tokens, heads, hd), 821), rand((cap, kv, hd), 822), rand((cap, kv, hd), 823)
+    assert_close(hip_ops.attention(q, k, v, start, "f32"), orc.attention(q, k, v, start), 2e-6, 1e-5, "f32 cache")
+    assert_close(hip_ops.attention(q, k, v, start, "f16"), orc.attention(q, _f16(k), _f16(v), start), 2e-5, 1e-4,
+                 "f16 cache")
+
+
 @pytest.mark.parametrize("tokens,start,hd", [(20, 0, 64), (16, 37, 32), (37, 5, 128)])
 def test_float32_attention_keeps_later_values_from_earlier_queries(hip_ops, tokens, start, hd):
     """A value that is an infinity or NaN reaches the queries that see its key and no others."""
@@ -68,3 +81,17 @@ def test_float32_attention_keeps_later_values_from_earlier_queries(hip_ops, toke
     assert np.array_equal(np.isfinite(got), np.isfinite(want))
     seen = np.isfinite(want)
     assert_close(got[seen], want[seen], 2e-6, 1e-5, "finite outputs")
+
+
+@pytest.mark.parametrize("cache", ["f32", "f16"])
+@pytest.mark.parametrize("tokens,start,hd", [(11, 0, 64), (11, 150, 64), (15, 401, 128)])
+def test_few_queries_do_not_see_later_values(hip_ops, tokens, start, hd, cache):
+    """The same for calls of 2 to 15 tokens, over both caches and with four, eight and sixteen waves."""
+    cap = start + tokens
+    q, k, v = rand((tokens, 4, hd), 831), rand((cap, 2, hd), 832), rand((cap, 2, hd), 833)
+    v[start + 4, 0, 3], v[start + tokens - 2, 1, hd - 1] = np.inf, np.nan
+    got = hip_ops.attention(q, k, v, start, cache)
+    want = orc.attention(q, k, v, start) if cache == "f32" else orc.attention(q, _f16(k), _f16(v), start)
+    assert np.array_equal(np.isfinite(got), np.isfinite(want))
+    seen = np.isfinite(want)
+    assert_close(got[seen], want[seen], *((2e-6, 1e-5) if cache == "f32" else (2e-5, 1e-4)), "finite outputs")
