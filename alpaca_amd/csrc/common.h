@@ -323,12 +323,15 @@ hipError_t launch_gemm_qkv_rope(const f16* x, const f16* xlo, int ldx, int m, co
 // pipelined tiles are faster.  The input is the activations' f16 terms (x,
 // xlo) or, with `gain` set, the float32 rows xf (row stride ldx), RMS-normalised
 // on the way in and rounded to the same terms (second terms as lo_row0 /
-// lo_col0 say; a lo_row0 past the last row: none).  `rope` for GEMM_QKV_ROPE.
+// lo_col0 say; a lo_row0 past the last row: none).  With `f32` set the rows xf
+// (normalised if `gain` is) enter as float32, without rounding, and results are
+// written as float32 (y; q of GEMM_QKV_ROPE too).  `rope` for GEMM_QKV_ROPE.
 // launch_gemm_mfma and launch_gemm_qkv_rope take it where it applies.
 struct SmallGemmInput {
     const f16* x = nullptr;
     const f16* xlo = nullptr;
     const float* xf = nullptr;
+    bool f32 = false;
     const float* gain = nullptr;
     float eps = 0.f;
     int ldx = 0;

@@ -1,9 +1,10 @@
-// Quants to exact f16 MFMA fragments, shared by the prefill GEMMs.
+// Quants to exact f16 or bf16 MFMA fragments, shared by the prefill GEMMs.
 #pragma once
 
 #include "common.h"
 
 typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
 __device__ __forceinline__ uint32_t as_u32(h2 v) { return __builtin_bit_cast(uint32_t, v); }
 
@@ -19,4 +20,19 @@ __device__ __forceinline__ void nib4_to_f16(uint32_t nib, uint32_t& o0, uint32_t
     const h2 bias = {(f16)1032.0f, (f16)1032.0f};
     o0 = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, nib, 0x04010400u)) - bias);
     o1 = as_u32(as_h2(__builtin_amdgcn_perm(0x64646464u, nib, 0x04030402u)) - bias);
+}
+// The same as bf16 pairs: the top halves of their float32 values (exact).
+__device__ __forceinline__ void int8x4_to_bf16(uint32_t w, uint32_t& o0, uint32_t& o1) {
+    float f[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) f[e] = (float)(int8_t)(w >> (8 * e));
+    o0 = __builtin_amdgcn_perm(__float_as_uint(f[1]), __float_as_uint(f[0]), 0x07060302u);
+    o1 = __builtin_amdgcn_perm(__float_as_uint(f[3]), __float_as_uint(f[2]), 0x07060302u);
+}
+__device__ __forceinline__ void nib4_to_bf16(uint32_t nib, uint32_t& o0, uint32_t& o1) {
+    float f[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) f[e] = (float)((nib >> (8 * e)) & 255u) - 8.0f;
+    o0 = __builtin_amdgcn_perm(__float_as_uint(f[1]), __float_as_uint(f[0]), 0x07060302u);
+    o1 = __builtin_amdgcn_perm(__float_as_uint(f[3]), __float_as_uint(f[2]), 0x07060302u);
 }

@@ -25,6 +25,23 @@
 // and each block's float32 MFMA result is scaled by d before it is added.
 // Each wave adds its blocks in K order and the waves' sums are added in wave
 // order, so an output depends on K and NW only, not on the tile or the grid.
+//
+// F32 (calls of 2 to 15 tokens): float32 activations without loss.  A float32 is
+// the exact sum of three bf16 terms (24 significant bits in three times 8, the
+// exponent range the same), a quant or nibble is one and an f16 weight two, so
+// bf16 MFMA products of the terms are the float32 products themselves, summed in
+// float32, smallest terms first.  The rows stay float32 in HBM and LDS (the bytes
+// of two f16 terms) and a lane takes a fragment apart as it reads it: with K split
+// over the waves each element is taken apart once a workgroup.  (An infinity gives
+// NaN one product earlier than the next RMSNorm would.)  Of a layer whose logits
+// pass gate+up, down and the head, relative to 64 bits: 1.8e-7 to 2.5e-7 at every
+// shape and format below, for rows from 1e-3 and products from 1e-6 to past 65,504;
+// the float32 GEMM on the VALU 2.7e-7 to 4.3e-7 (Q8_0, Q4_0) and 0.9e-6 to 2.0e-6
+// (F16).  11 rows, us a launch, VALU / this (QKV and gate+up of the first two with
+// their RMSNorm, another 2.7 before the VALU's):
+//   135M shape, Q8_0   QKV  5.3 / 5.8   Wo  5.2 / 4.1   gate+up 11.7 /  6.2   down  8.4 /  5.2
+//   360M shape, Q4_0   QKV  6.7 / 6.6   Wo  5.2 / 4.7   gate+up 14.1 /  7.5   down 10.2 /  7.0
+//   1.7B shape, Q8_0   QKV 28.0 / 8.9   Wo 18.3 / 6.3   gate+up 57.0 / 13.6   down 59.2 / 14.0
 #include "common.h"
 #include "gemm_frag.h"
 
@@ -56,9 +73,9 @@ constexpr int SK = 64;  // K per stage (two quant blocks)
 constexpr int kNormV = 4;  // float4 per lane of a normalised row (K <= 1,024)
 
 // One wave's stage buffer: the activations' rows (128 B, the second term's
-// after the first's; absent with NORM, whose rows are shared), each matrix's
-// weight rows, each matrix's scale pairs.
-template <int FMT, int TM, int TN, int NB, bool NORM>
+// after the first's, or 256 B of float32; absent with NORM, whose rows are
+// shared), each matrix's weight rows, each matrix's scale pairs.
+template <int FMT, int TM, int TN, int NB, bool NORM, bool F32>
 struct SmallStage {
     static constexpr int BROW = FMT == DT_Q8_0 ? 64 : FMT == DT_Q4_0 ? 32 : 128;
     static constexpr int A_LO = 16 * TM * 128;
@@ -67,28 +84,58 @@ struct SmallStage {
     static constexpr int BYTES = S_OFF + (FMT == DT_F16 ? 0 : NB * 16 * TN * 4);
     // DMA instructions of a stage, without the activations' second term
     static constexpr int B_I = FMT == DT_Q8_0 ? TN : FMT == DT_Q4_0 ? (TN + 1) / 2 : 2 * TN;
-    static constexpr int A_I = NORM ? 0 : 2 * TM;
+    static constexpr int A_I = NORM ? 0 : F32 ? 4 * TM : 2 * TM;
     static constexpr int PER = A_I + NB * (B_I + (FMT == DT_F16 ? 0 : 1));
 };
 
 // LDS row pitch of the normalised activations: 16 bytes past a multiple of 256,
 // so the 16 rows of a fragment read fall in 16 distinct 16-byte bank groups.
-__host__ __device__ constexpr int norm_pitch(int K) { return (2 * K + 255) / 256 * 256 + 16; }
+__host__ __device__ constexpr int norm_pitch(int row_bytes) { return (row_bytes + 255) / 256 * 256 + 16; }
 
-template <int FMT, int MODE, int TM, int TN, int NW, int D, int NV>
+// Bytes of the tile's normalised rows: two f16 planes or one of float32.
+template <int TM, bool F32>
+__host__ __device__ constexpr int norm_bytes(int K) {
+    return 16 * TM * (F32 ? norm_pitch(4 * K) : 2 * norm_pitch(2 * K));
+}
+
+template <int FMT, int MODE, int TM, int TN, int NW, int D, int NV, bool F32>
 constexpr size_t small_lds(int K) {
     constexpr int NB = MODE == GEMM_SWIGLU ? 2 : 1;
-    const size_t ring = (size_t)NW * D * SmallStage<FMT, TM, TN, NB, (NV > 0)>::BYTES;
-    const size_t rows = NV > 0 ? (size_t)2 * 16 * TM * norm_pitch(K) : 0;
+    const size_t ring = (size_t)NW * D * SmallStage<FMT, TM, TN, NB, (NV > 0), F32>::BYTES;
+    const size_t rows = NV > 0 ? (size_t)norm_bytes<TM, F32>(K) : 0;
     return std::max(ring + rows, (size_t)NW * NB * TM * TN * 1024);  // the waves' accumulators reuse it
 }
 
-template <int FMT, int MODE, int TM, int TN, int NW, int D, int NV>
+// The top halves of two floats as a bf16 pair.
+__device__ __forceinline__ uint32_t bf16_tops(float a, float b) {
+    return __builtin_amdgcn_perm(__float_as_uint(b), __float_as_uint(a), 0x07060302u);
+}
+__device__ __forceinline__ float bf16_top(float a) { return __uint_as_float(__float_as_uint(a) & 0xFFFF0000u); }
+__device__ __forceinline__ bf16x8 as_bf16x8(const uint32_t (&o)[4]) {
+    return __builtin_bit_cast(bf16x8, make_uint4(o[0], o[1], o[2], o[3]));
+}
+// Eight floats as N bf16 terms, largest first: each the top half of what the ones
+// before it leave (exact differences; three hold every float32, two every f16).
+template <int N>
+__device__ __forceinline__ void bf16_split(float (&x)[8], bf16x8 (&t)[N]) {
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+        uint32_t o[4];
+#pragma unroll
+        for (int e = 0; e < 4; e++) o[e] = bf16_tops(x[2 * e], x[2 * e + 1]);
+        t[n] = as_bf16x8(o);
+        if (n + 1 < N)
+#pragma unroll
+            for (int e = 0; e < 8; e++) x[e] -= bf16_top(x[e]);
+    }
+}
+
+template <int FMT, int MODE, int TM, int TN, int NW, int D, int NV, bool F32>
 __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(SmallArgs p) {
     constexpr int NB = MODE == GEMM_SWIGLU ? 2 : 1;
     constexpr int F = TM * TN;  // 16x16 fragments per matrix
     constexpr bool QUANT = FMT != DT_F16, NORM = NV > 0;
-    using L = SmallStage<FMT, TM, TN, NB, NORM>;
+    using L = SmallStage<FMT, TM, TN, NB, NORM, F32>;
     extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
 
     const int K = p.w.cols, N = p.w.rows, M = p.M, nb = K >> 5, nk = K / SK, spitch = stage_scale_pitch(N);
@@ -101,17 +148,22 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(SmallArgs p) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int per = (nk + NW - 1) / NW, k0 = wave * per, cnt = max(0, min(nk - k0, per));  // this wave's stages
     const bool use_lo = (NORM || p.in.xlo) && (m0 + 16 * TM > p.lo_row0 || n0 + 16 * TN > p.lo_col0);
-    const int pitch = norm_pitch(K);
-    uint8_t* const rows = smem;  // NORM: the tile's normalised rows, first terms then second
-    uint8_t* const ring = smem + (NORM ? 2 * 16 * TM * pitch : 0) + wave * D * L::BYTES;
+    const int pitch = norm_pitch(F32 ? 4 * K : 2 * K);
+    uint8_t* const rows = smem;  // NORM: the tile's normalised rows, first terms then second, or float32
+    uint8_t* const ring = smem + (NORM ? norm_bytes<TM, F32>(K) : 0) + wave * D * L::BYTES;
 
     // Per-lane DMA source offsets (rows past the edges clamped to the last).
-    uint32_t aoff[NORM ? 1 : 2 * TM], boff[L::B_I], soff = 0;
+    uint32_t aoff[NORM ? 1 : L::A_I], boff[L::B_I], soff = 0;
     if constexpr (!NORM) {
 #pragma unroll
-        for (int i = 0; i < 2 * TM; i++) {
-            const int r = 8 * i + (lane >> 3), c = (lane & 7) ^ swz_a(r);
-            aoff[i] = (uint32_t)((min(m0 + r, M - 1) * p.in.ldx + c * 8) * 2);
+        for (int i = 0; i < L::A_I; i++) {
+            if constexpr (F32) {
+                const int r = 4 * i + (lane >> 4), c = (lane & 15) ^ (r & 15);
+                aoff[i] = (uint32_t)((min(m0 + r, M - 1) * p.in.ldx + c * 4) * 4);
+            } else {
+                const int r = 8 * i + (lane >> 3), c = (lane & 7) ^ swz_a(r);
+                aoff[i] = (uint32_t)((min(m0 + r, M - 1) * p.in.ldx + c * 8) * 2);
+            }
         }
     }
 #pragma unroll
@@ -137,8 +189,9 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(SmallArgs p) {
         const int kt = __builtin_amdgcn_readfirstlane(kt_);
         if constexpr (!NORM) {
 #pragma unroll
-            for (int i = 0; i < 2 * TM; i++) {
-                dma16s(p.in.x + kt * SK, aoff[i], sg + i * 1024);
+            for (int i = 0; i < L::A_I; i++) {
+                if constexpr (F32) dma16s(p.in.xf + kt * SK, aoff[i], sg + i * 1024);
+                else dma16s(p.in.x + kt * SK, aoff[i], sg + i * 1024);
                 if constexpr (TT) dma16s(p.in.xlo + kt * SK, aoff[i], sg + L::A_LO + i * 1024);
             }
         }
@@ -200,10 +253,23 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(SmallArgs p) {
 #pragma unroll
             for (int kk = 0; kk < 2; kk++) {
                 f16x8 ah[TM], al[TT ? TM : 1];
+                bf16x8 ax[F32 ? TM : 1][3];
 #pragma unroll
                 for (int i = 0; i < TM; i++) {
                     const int r = 16 * i + l16;
-                    if constexpr (NORM) {
+                    if constexpr (F32) {
+                        float xv[8];
+#pragma unroll
+                        for (int h = 0; h < 2; h++) {
+                            const uint8_t* a =
+                                NORM ? rows + r * pitch + (kt * SK + 32 * kk + 8 * g + 4 * h) * 4
+                                     : sg + r * 256 + ((8 * kk + 2 * g + h) ^ (r & 15)) * 16;
+                            const f32x4 v = *(const f32x4*)a;
+#pragma unroll
+                            for (int e = 0; e < 4; e++) xv[4 * h + e] = v[e];
+                        }
+                        bf16_split(xv, ax[i]);
+                    } else if constexpr (NORM) {
                         const uint8_t* a = rows + r * pitch + (kt * SK + 32 * kk + 8 * g) * 2;
                         ah[i] = *(const f16x8*)a;
                         if constexpr (TT) al[i] = *(const f16x8*)(a + 16 * TM * pitch);
@@ -220,31 +286,61 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(SmallArgs p) {
                         const int r = 16 * j + l16;
                         const uint8_t* bq = sg + L::B_OFF + mat * 16 * TN * L::BROW;
                         f16x8 bf;
-                        float d = 0.f;
+                        bf16x8 bx[FMT == DT_F16 ? 2 : 1];
+                        float d = 1.f;
                         if constexpr (QUANT) {
                             uint32_t o[4];
                             if constexpr (FMT == DT_Q8_0) {
                                 const int u = 4 * kk + g;
                                 const uint2 raw = *(const uint2*)(bq + r * 64 + ((u >> 1) ^ swz_q8(r)) * 16 + (u & 1) * 8);
-                                int8x4_to_f16(raw.x, o[0], o[1]);
-                                int8x4_to_f16(raw.y, o[2], o[3]);
+                                if constexpr (F32) {
+                                    int8x4_to_bf16(raw.x, o[0], o[1]);
+                                    int8x4_to_bf16(raw.y, o[2], o[3]);
+                                } else {
+                                    int8x4_to_f16(raw.x, o[0], o[1]);
+                                    int8x4_to_f16(raw.y, o[2], o[3]);
+                                }
                             } else {
                                 const uint2 raw = *(const uint2*)(bq + r * 32 + (kk ^ swz_q4(r)) * 16 + (g & 1) * 8);
                                 const int sh = (g >> 1) * 4;  // low nibbles: elements 0..15, high: 16..31
-                                nib4_to_f16((raw.x >> sh) & 0x0F0F0F0Fu, o[0], o[1]);
-                                nib4_to_f16((raw.y >> sh) & 0x0F0F0F0Fu, o[2], o[3]);
+                                const uint32_t n0_ = (raw.x >> sh) & 0x0F0F0F0Fu, n1_ = (raw.y >> sh) & 0x0F0F0F0Fu;
+                                if constexpr (F32) {
+                                    nib4_to_bf16(n0_, o[0], o[1]);
+                                    nib4_to_bf16(n1_, o[2], o[3]);
+                                } else {
+                                    nib4_to_f16(n0_, o[0], o[1]);
+                                    nib4_to_f16(n1_, o[2], o[3]);
+                                }
                             }
-                            bf = __builtin_bit_cast(f16x8, make_uint4(o[0], o[1], o[2], o[3]));
+                            if constexpr (F32) bx[0] = as_bf16x8(o);
+                            else bf = __builtin_bit_cast(f16x8, make_uint4(o[0], o[1], o[2], o[3]));
                             d = (float)*(const f16*)(sg + L::S_OFF + (mat * 16 * TN + r) * 4 + kk * 2);
                         } else {
                             bf = *(const f16x8*)(bq + r * 128 + ((4 * kk + g) ^ swz_a(r)) * 16);
+                            if constexpr (F32) {
+                                float wv[8];
+#pragma unroll
+                                for (int e = 0; e < 8; e++) wv[e] = (float)bf[e];
+                                bf16_split(wv, bx);
+                            }
                         }
 #pragma unroll
                         for (int i = 0; i < TM; i++) {
-                            f32x4 c = QUANT ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[mat][i][j];
-                            c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bf, c, 0, 0, 0);
-                            if constexpr (TT) c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], bf, c, 0, 0, 0);
+                            f32x4 c = QUANT || F32 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[mat][i][j];
+                            if constexpr (F32) {
+                                constexpr int WT = FMT == DT_F16 ? 2 : 1;
+#pragma unroll
+                                for (int t = WT + 1; t >= 0; t--)  // terms of order t: x's n-th by w's (t - n)-th
+#pragma unroll
+                                    for (int n = 2; n >= 0; n--)
+                                        if (t - n >= 0 && t - n < WT)
+                                            c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ax[i][n], bx[t - n], c, 0, 0, 0);
+                            } else {
+                                c = __builtin_amdgcn_mfma_f32_16x16x32_f16(ah[i], bf, c, 0, 0, 0);
+                                if constexpr (TT) c = __builtin_amdgcn_mfma_f32_16x16x32_f16(al[i], bf, c, 0, 0, 0);
+                            }
                             if constexpr (QUANT) acc[mat][i][j] += d * c;
+                            else if constexpr (F32) acc[mat][i][j] += c;
                             else acc[mat][i][j] = c;
                         }
                     }
@@ -288,6 +384,10 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(SmallArgs p) {
                     const float4 gn = gv[k];
                     const float4 yv = {(v[q][k].x * scale) * gn.x, (v[q][k].y * scale) * gn.y,
                                        (v[q][k].z * scale) * gn.z, (v[q][k].w * scale) * gn.w};
+                    if constexpr (F32) {
+                        *(f32x4*)(rows + row * pitch + 16 * i) = f32x4{yv.x, yv.y, yv.z, yv.w};
+                        continue;
+                    }
                     const f16x4 hi = {(f16)yv.x, (f16)yv.y, (f16)yv.z, (f16)yv.w};
                     *(f16x4*)(rows + row * pitch + 8 * i) = hi;
                     if constexpr (TT)
@@ -312,8 +412,12 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(SmallArgs p) {
             }
         }
     };
-    if (use_lo) run(std::true_type{});
-    else run(std::false_type{});
+    if constexpr (F32) {
+        run(std::false_type{});
+    } else {
+        if (use_lo) run(std::true_type{});
+        else run(std::false_type{});
+    }
 
     // No DMA may still be writing LDS, and every wave is done reading it.
     wait_stage_barrier<0>();
@@ -361,8 +465,12 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(SmallArgs p) {
                 const f16 ho = (f16)out;
                 if (region == 0) {
                     const int64_t at = (int64_t)m * p.ldy + n;
-                    p.yh[at] = ho;
-                    if (p.yhlo && m >= p.lo_out_row0) p.yhlo[at] = (f16)(out - (float)ho);
+                    if constexpr (F32) {
+                        p.y[at] = out;
+                    } else {
+                        p.yh[at] = ho;
+                        if (p.yhlo && m >= p.lo_out_row0) p.yhlo[at] = (f16)(out - (float)ho);
+                    }
                 } else {
                     f16* c = region == 1 ? o.kc : o.vc;
                     c[((int64_t)(cn / o.hd) * o.capacity + o.pos + m) * o.hd + cn % o.hd] = ho;
@@ -381,21 +489,25 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(SmallArgs p) {
                     p.y[at] = pre[k][r][0] + s[0][r];
                 } else {
                     const float gt = s[0][r];
-                    const float v = (gt / (1.0f + __expf(-gt))) * s[NB - 1][r];
-                    const f16 hv = (f16)v;
-                    p.yh[at] = hv;
-                    if (p.yhlo && m >= p.lo_out_row0) p.yhlo[at] = (f16)(v - (float)hv);
+                    if constexpr (F32) {
+                        p.y[at] = (gt / (1.0f + expf(-gt))) * s[NB - 1][r];
+                    } else {
+                        const float v = (gt / (1.0f + __expf(-gt))) * s[NB - 1][r];
+                        const f16 hv = (f16)v;
+                        p.yh[at] = hv;
+                        if (p.yhlo && m >= p.lo_out_row0) p.yhlo[at] = (f16)(v - (float)hv);
+                    }
                 }
             }
         }
     }
 }
 
-template <int FMT, int MODE, int TM, int TN, int NW, int D, int NV>
+template <int FMT, int MODE, int TM, int TN, int NW, int D, int NV, bool F32>
 hipError_t run_small(const SmallArgs& a, hipStream_t st) {
     const int tiles = ((a.M + 16 * TM - 1) / (16 * TM)) * ((a.w.rows + 16 * TN - 1) / (16 * TN));
-    const size_t lds = small_lds<FMT, MODE, TM, TN, NW, D, NV>(a.w.cols);
-    auto* kernel = small_gemm_kernel<FMT, MODE, TM, TN, NW, D, NV>;
+    const size_t lds = small_lds<FMT, MODE, TM, TN, NW, D, NV, F32>(a.w.cols);
+    auto* kernel = small_gemm_kernel<FMT, MODE, TM, TN, NW, D, NV, F32>;
     static const hipError_t attr =
         hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10);
     if (attr != hipSuccess) return attr;
@@ -405,38 +517,42 @@ hipError_t run_small(const SmallArgs& a, hipStream_t st) {
 
 // Tile families, smallest first.  F16 weight stages are twice the size, and
 // SwiGLU keeps two of them: the largest tile's then leave room for four waves.
-template <int FMT, int MODE, int NV>
+// Normalised rows and float32 ones take the two smallest.
+template <int FMT, int MODE, int NV, bool F32>
 hipError_t run_family(int family, const SmallArgs& a, hipStream_t st) {
     constexpr int DW = FMT == DT_F16 && MODE == GEMM_SWIGLU ? 1 : 2;
     switch (family) {
-    case 0: return run_small<FMT, MODE, 1, 1, 8, 2, NV>(a, st);
-    case 1: return run_small<FMT, MODE, 1, 2, 8, DW, NV>(a, st);
+    case 0: return run_small<FMT, MODE, 1, 1, 8, 2, NV, F32>(a, st);
+    case 1: return run_small<FMT, MODE, 1, 2, 8, DW, NV, F32>(a, st);
     case 2:
-        if constexpr (NV == 0) return run_small<FMT, MODE, 2, 2, 8, 1, 0>(a, st);
+        if constexpr (NV == 0 && !F32) return run_small<FMT, MODE, 2, 2, 8, 1, 0, false>(a, st);
         break;
     case 3:
-        if constexpr (NV == 0) return run_small<FMT, MODE, 2, 4, DW == 1 ? 4 : 8, 1, 0>(a, st);
+        if constexpr (NV == 0 && !F32) return run_small<FMT, MODE, 2, 4, DW == 1 ? 4 : 8, 1, 0, false>(a, st);
         break;
     }
     return hipErrorNotSupported;
 }
 
-template <int FMT, int NV>
+template <int FMT, int NV, bool F32>
 hipError_t run_mode(int mode, int family, const SmallArgs& a, hipStream_t st) {
     switch (mode) {
-    case GEMM_STORE: return run_family<FMT, GEMM_STORE, NV>(family, a, st);
-    case GEMM_SWIGLU: return run_family<FMT, GEMM_SWIGLU, NV>(family, a, st);
-    case GEMM_QKV_ROPE: return run_family<FMT, GEMM_QKV_ROPE, NV>(family, a, st);
+    case GEMM_STORE: return run_family<FMT, GEMM_STORE, NV, F32>(family, a, st);
+    case GEMM_SWIGLU: return run_family<FMT, GEMM_SWIGLU, NV, F32>(family, a, st);
+    case GEMM_QKV_ROPE: return run_family<FMT, GEMM_QKV_ROPE, NV, F32>(family, a, st);
     case GEMM_ACC:
-        if constexpr (NV == 0) return run_family<FMT, GEMM_ACC, 0>(family, a, st);
+        if constexpr (NV == 0) return run_family<FMT, GEMM_ACC, 0, F32>(family, a, st);
         break;
     }
     return hipErrorNotSupported;
 }
 
 template <int FMT>
-hipError_t run_norm(bool norm, int mode, int family, const SmallArgs& a, hipStream_t st) {
-    return norm ? run_mode<FMT, kNormV>(mode, family, a, st) : run_mode<FMT, 0>(mode, family, a, st);
+hipError_t run_input(int mode, int family, const SmallArgs& a, hipStream_t st) {
+    const bool norm = a.in.gain != nullptr;
+    if (a.in.f32)
+        return norm ? run_mode<FMT, kNormV, true>(mode, family, a, st) : run_mode<FMT, 0, true>(mode, family, a, st);
+    return norm ? run_mode<FMT, kNormV, false>(mode, family, a, st) : run_mode<FMT, 0, false>(mode, family, a, st);
 }
 
 int device_cus() {
@@ -478,13 +594,19 @@ int device_cus() {
 // streams, the pipelined tiles keep every shape: they sum K in one order
 // whatever the tile, so a split prompt's one-term rows are those of an unsplit
 // one.
-static int small_family(int m, const DevMatrix& w, bool norm) {
-    const char* forced = std::getenv("ALPACA_HIP_GEMM_TILE");  // a pipelined tile, or none (tuning and tests)
-    if (m >= 768 || (forced && *forced)) return -1;
+// Float32 rows (fewer than 16) have no pipelined form: the 16x32 tiles take the
+// larger grids too.
+static int small_family(int m, const DevMatrix& w, const SmallGemmInput& in) {
     static const int tile[4][2] = {{16, 16}, {16, 32}, {32, 32}, {32, 64}};
     const int64_t cus = device_cus();
-    for (int f = 0; f < (norm ? 2 : 4); f++)
-        if ((int64_t)((m + tile[f][0] - 1) / tile[f][0]) * ((w.rows + tile[f][1] - 1) / tile[f][1]) <= cus) return f;
+    auto fits = [&](int f) {
+        return (int64_t)((m + tile[f][0] - 1) / tile[f][0]) * ((w.rows + tile[f][1] - 1) / tile[f][1]) <= cus;
+    };
+    if (in.f32) return fits(0) ? 0 : 1;
+    const char* forced = std::getenv("ALPACA_HIP_GEMM_TILE");  // a pipelined tile, or none (tuning and tests)
+    if (m >= 768 || (forced && *forced)) return -1;
+    for (int f = 0; f < (in.gain ? 2 : 4); f++)
+        if (fits(f)) return f;
     return -1;
 }
 
@@ -494,10 +616,9 @@ bool gemm_small_takes(const SmallGemmInput& in, int m, const DevMatrix& w, const
     // that 32-bit byte offsets reach
     if (w.cols % SK || in.ldx % 8 || (quant && (!w.s2 || (w_up && !w_up->s2)))) return false;
     if ((int64_t)w.rows * w.cols * 2 > INT32_MAX || (int64_t)m * in.ldx * 4 > INT32_MAX) return false;
-    if (norm ? (w.cols > 256 * kNormV || ((uintptr_t)in.xf & 15) || ((uintptr_t)in.gain & 15))
-             : (((uintptr_t)in.x & 15) || ((uintptr_t)in.xlo & 15)))
-        return false;
-    return small_family(m, w, norm) >= 0;
+    if (norm && (w.cols > 256 * kNormV || ((uintptr_t)in.gain & 15))) return false;
+    if (norm || in.f32 ? ((uintptr_t)in.xf & 15) != 0 : (((uintptr_t)in.x | (uintptr_t)in.xlo) & 15) != 0) return false;
+    return small_family(m, w, in) >= 0;
 }
 
 hipError_t launch_gemm_small(const SmallGemmInput& in, int m, const DevMatrix& w, const DevMatrix* w_up, float* y,
@@ -508,8 +629,7 @@ hipError_t launch_gemm_small(const SmallGemmInput& in, int m, const DevMatrix& w
     if (mode == GEMM_QKV_ROPE &&
         (!rope || rope->hd % 16 || w.rows != (rope->heads + 2 * rope->kv_heads) * rope->hd))
         return hipErrorInvalidValue;  // a fragment must not straddle a head
-    const bool norm = in.gain != nullptr;
-    const int family = small_family(m, w, norm);
+    const int family = small_family(m, w, in);
     SmallArgs a;
     a.in = in;
     a.M = m;
@@ -528,8 +648,8 @@ hipError_t launch_gemm_small(const SmallGemmInput& in, int m, const DevMatrix& w
     const int64_t wb = (int64_t)w.rows * (w.dtype == DT_Q8_0 ? 34 : w.dtype == DT_Q4_0 ? 18 : 64) * (w_up ? 2 : 1);
     a.by_cols = wb >= (int64_t)m * 128;
     switch (w.dtype) {
-    case DT_Q8_0: return run_norm<DT_Q8_0>(norm, mode, family, a, st);
-    case DT_Q4_0: return run_norm<DT_Q4_0>(norm, mode, family, a, st);
-    default: return run_norm<DT_F16>(norm, mode, family, a, st);
+    case DT_Q8_0: return run_input<DT_Q8_0>(mode, family, a, st);
+    case DT_Q4_0: return run_input<DT_Q4_0>(mode, family, a, st);
+    default: return run_input<DT_F16>(mode, family, a, st);
     }
 }

@@ -1380,14 +1380,8 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
     // and 64-query blocks then either lie wholly in that range or wholly
     // before it, so the same rows take two terms whatever tile a GEMM picks.
     // With lo_all_rows every row takes them.
-    // Below 16 rows every operand of every session takes its second term: such
-    // a call's activations keep float32 grade whatever the session's precision
-    // (one MFMA tile of rows costs the same with one term or two).
-    const bool few = n < 16;
-    // ... and its weights: the quants, not the f16 copies of the prefill weight cache
-    auto pre = [&](const OwnedMatrix& w, const OwnedMatrix& h) -> const DevMatrix& { return few ? w.m : L.pre(w, h); };
-    const int lo = few ? kLoAll : s->two_term ? s->lo_terms : 0;
-    const bool all = s->lo_all_rows || few;
+    const int lo = s->two_term ? s->lo_terms : 0;
+    const bool all = s->lo_all_rows;
     const int tail0 = all ? 0 : last ? (n - 1) / 256 * 256 : n;
     const int lo_tile = tail0;
     auto want = [&](int bit) { return (lo & bit) && (all || last); };
@@ -1409,7 +1403,7 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
         return in;
     };
     const int none = 1 << 30;  // a first row past the last: no second terms
-    const DevMatrix& wqkv = pre(L.qkv, L.qkv16);
+    const DevMatrix& wqkv = L.pre(L.qkv, L.qkv16);
     hipError_t fused = hipErrorNotSupported;
     const bool rope_fused = flash && s->fuse_qkv_rope;
     QkvRope o;
@@ -1492,7 +1486,7 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
     const int side = (!all && last && tail0 > 0) ? last_row_gemv_mask(L, n) : 0;
     const int64_t lr = n - 1;  // the last row
     s->stage("attn out projection (+residual)");
-    const DevMatrix& wo = pre(L.wo, L.wo16);
+    const DevMatrix& wo = L.pre(L.wo, L.wo16);
     if ((side & kSideWo) && ctxhlo) {
         LAUNCH(launch_gemm_mfma(ctxh, nullptr, QW, n - 1, wo, nullptr, x, nullptr, nullptr, H, GEMM_ACC, st));
         LAUNCH(launch_gemv_pair(wo, nullptr, ctxh + lr * QW, ctxhlo + lr * QW, x + lr * H, nullptr, nullptr, GEMV_ADD,
@@ -1500,7 +1494,7 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
     } else {
         LAUNCH(launch_gemm_mfma(ctxh, ctxhlo, QW, n, wo, nullptr, x, nullptr, nullptr, H, GEMM_ACC, st, lo_tile));
     }
-    const DevMatrix &wg = pre(L.gate, L.gate16), &wu = pre(L.up, L.up16);
+    const DevMatrix &wg = L.pre(L.gate, L.gate16), &wu = L.pre(L.up, L.up16);
     const bool side_gu = (side & kSideGateUp) && xhlo_ffn && ffnhlo;
     const SmallGemmInput ffn_in = normed_row(L.ffn_norm);
     const bool ffn_normed = !side_gu && gemm_small_takes(ffn_in, n, wg, &wu);
@@ -1520,7 +1514,7 @@ static int encode_mfma_layer(ahip_session* s, int li, int row0, int n, int pos, 
         LAUNCH(launch_gemm_mfma(xh, xhlo_ffn, H, n, wg, &wu, nullptr, ffnh, ffnhlo, F, GEMM_SWIGLU, st, lo_tile, tail0));
     }
     s->stage("ffn down (+residual)");
-    const DevMatrix& wd = pre(L.down, L.down16);
+    const DevMatrix& wd = L.pre(L.down, L.down16);
     if ((side & kSideDown) && ffnhlo) {
         LAUNCH(launch_gemm_mfma(ffnh, nullptr, F, n - 1, wd, nullptr, x, nullptr, nullptr, H, GEMM_ACC, st));
         LAUNCH(launch_gemv_pair(wd, nullptr, ffnh + lr * F, ffnhlo + lr * F, x + lr * H, nullptr, nullptr, GEMV_ADD,
@@ -1616,13 +1610,12 @@ static int encode_chunk(ahip_session* s, const int32_t* dtok, int n, int pos, bo
     float* x = s->x.as<float>();
     float* qkv = s->qkv.as<float>();
     const float2* rope = m->rope.as<float2>();
-    const bool flash_fits = s->fast && !s->prefill_generic_attention && s->kv_f16 && (hd == 64 || hd == 128);
-    // (below 16 rows every operand takes its second term, encode_mfma_layer; without the flash
-    // kernel those calls stay on the float32 kernels)
-    const bool mfma = s->fast && !s->prefill_f32_gemm && (n >= 16 || flash_fits);
-    // the flash kernel takes q and P as f16 terms and multiplies every value of a key block, also
-    // those of later keys, by p = 0: below 16 rows attention stays on the float32 kernel
-    const bool flash = flash_fits && n >= 16;
+    const bool mfma = s->fast && n >= 16 && !s->prefill_f32_gemm;
+    const bool flash = s->fast && n >= 16 && !s->prefill_generic_attention && s->kv_f16 && (hd == 64 || hd == 128);
+    // Calls of 2 to 15 tokens keep float32 activations in every mode: the fast modes'
+    // on bf16 MFMA without loss (launch_gemm_small), summed in its order; with a
+    // float32 cache, the setting that numerics are checked in, in the reference's.
+    const bool few = s->fast && n < 16 && s->kv_f16 && !s->prefill_f32_gemm;
     if (mfma && n >= env_int("ALPACA_HIP_SPLIT_MIN", kSplitPrefillMin) && !s->profiling && env_int("ALPACA_HIP_PREFILL_STREAMS", 2) >= 2 &&
         prefill_split_pays(n, QW + 2 * KW)) {
         if (!s->part_stream[1]) s->part_stream[1] = split_stream_acquire(m->device);
@@ -1644,14 +1637,48 @@ static int encode_chunk(ahip_session* s, const int32_t* dtok, int n, int pos, bo
             if (int rc = encode_mfma_layer(s, li, 0, n, pos, flash, logits, st, nullptr, nullptr)) return rc;
         } else {
             float* xn = s->xn.as<float>();
-            s->stage("rmsnorm");
-            LAUNCH(launch_rmsnorm(x, L.attn_norm.as<float>(), xn, nullptr, nullptr, n, H, c.rms_norm_eps, st));
-            s->stage("qkv projections");
-            LAUNCH(launch_gemm_f32(xn, H, n, L.qkv.m, nullptr, qkv, LDQKV, GEMM_STORE, st));
-            s->stage("rope + kv store");
-            LAUNCH(launch_rope_store(qkv, LDQKV, n, c.head_count, c.kv_head_count, hd, pos, rope, 1, flash ? 0 : 1,
-                                     flash ? s->qh.as<f16>() : nullptr, flash ? qhlo : nullptr, kc, vc, s->kv_f16,
-                                     s->capacity, st));
+            QkvRope o;
+            o.rope = rope;
+            o.kc = (f16*)kc;
+            o.vc = (f16*)vc;
+            o.heads = c.head_count;
+            o.kv_heads = c.kv_head_count;
+            o.hd = hd;
+            o.pos = pos;
+            o.capacity = s->capacity;
+            bool roped = false;  // RoPE and the KV append were done in the GEMM
+            // float32 rows (through the RMSNorm if `gain` is set) by w
+            auto gemm = [&](const char* stage, const float* in, const DevBuf* gain, const DevMatrix& w,
+                            const DevMatrix* up, float* y, int ldy, int mode) -> hipError_t {
+                SmallGemmInput rows;
+                rows.f32 = true;
+                rows.ldx = w.cols;
+                rows.xf = in;
+                rows.eps = c.rms_norm_eps;
+                rows.gain = gain ? gain->as<float>() : nullptr;
+                if (gain && !(few && gemm_small_takes(rows, n, w, up))) {
+                    s->stage("rmsnorm");
+                    const hipError_t e =
+                        launch_rmsnorm(in, rows.gain, xn, nullptr, nullptr, n, w.cols, c.rms_norm_eps, st);
+                    if (e != hipSuccess) return e;
+                    rows.xf = xn;
+                    rows.gain = nullptr;
+                }
+                s->stage(stage);
+                if (few && gemm_small_takes(rows, n, w, up)) {
+                    roped = mode == GEMM_QKV_ROPE;
+                    return launch_gemm_small(rows, n, w, up, y, nullptr, nullptr, ldy, mode, &o, st, 0, 0);
+                }
+                return launch_gemm_f32(rows.xf, w.cols, n, w, up, y, ldy, mode == GEMM_QKV_ROPE ? GEMM_STORE : mode, st);
+            };
+            LAUNCH(gemm("qkv projections", x, &L.attn_norm, L.qkv.m, nullptr, qkv, LDQKV,
+                        s->fuse_qkv_rope ? GEMM_QKV_ROPE : GEMM_STORE));
+            if (!roped) {
+                s->stage("rope + kv store");
+                LAUNCH(launch_rope_store(qkv, LDQKV, n, c.head_count, c.kv_head_count, hd, pos, rope, 1, flash ? 0 : 1,
+                                         flash ? s->qh.as<f16>() : nullptr, flash ? qhlo : nullptr, kc, vc, s->kv_f16,
+                                         s->capacity, st));
+            }
             s->stage("attention");
             if (flash) {
                 LAUNCH(launch_flash_attention(s->qh.as<f16>(), qhlo, QW, (const f16*)kc, (const f16*)vc, s->capacity,
@@ -1661,14 +1688,9 @@ static int encode_chunk(ahip_session* s, const int32_t* dtok, int n, int pos, bo
                 LAUNCH(launch_attention_generic(qkv, LDQKV, kc, vc, s->kv_f16, s->capacity, n, c.head_count,
                                                 c.kv_head_count, hd, pos, 1, nullptr, s->ctx.as<float>(), st));
             }
-            s->stage("attn out projection (+residual)");
-            LAUNCH(launch_gemm_f32(s->ctx.as<float>(), QW, n, L.wo.m, nullptr, x, H, GEMM_ACC, st));
-            s->stage("rmsnorm");
-            LAUNCH(launch_rmsnorm(x, L.ffn_norm.as<float>(), xn, nullptr, nullptr, n, H, c.rms_norm_eps, st));
-            s->stage("ffn gate+up+silu");
-            LAUNCH(launch_gemm_f32(xn, H, n, L.gate.m, &L.up.m, s->ffn.as<float>(), F, GEMM_SWIGLU, st));
-            s->stage("ffn down (+residual)");
-            LAUNCH(launch_gemm_f32(s->ffn.as<float>(), F, n, L.down.m, nullptr, x, H, GEMM_ACC, st));
+            LAUNCH(gemm("attn out projection (+residual)", s->ctx.as<float>(), nullptr, L.wo.m, nullptr, x, H, GEMM_ACC));
+            LAUNCH(gemm("ffn gate+up+silu", x, &L.ffn_norm, L.gate.m, &L.up.m, s->ffn.as<float>(), F, GEMM_SWIGLU));
+            LAUNCH(gemm("ffn down (+residual)", s->ffn.as<float>(), nullptr, L.down.m, nullptr, x, H, GEMM_ACC));
         }
     }
     if (logits) {
