@@ -19,7 +19,8 @@
 //     draw, and one workgroup walks it.  The sums are associated by run rather
 //     than strictly left to right, so the token can differ from a strictly
 //     sequential sum only when u * sum falls within about 1e-16 (relative) of
-//     a boundary between two tokens.
+//     a boundary between two tokens.  A token whose probability is zero is never
+//     drawn, at such a boundary either.
 //   * top-k and/or top-p: one workgroup of 1024 threads takes candidates in the
 //     reference's order in windows of up to 1024, each the next smallest (key,
 //     index) pairs after the previous window.  The first window is gathered by
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(kRun) void sample_plain_kernel(SampleArgs a) {
             if (target < next) {
                 // this run's logits, one a thread: the waves' sums name the wave,
                 // its running sums the lane; sums that rounding leaves short pass
-                // on to the next wave or run
+                // on to the next token of a probability in the next wave or run
                 const int i = (r0 + c) * kRun + tid;
                 const double p = i < a.n ? prob(a.logits[i], top, t) : 0.0;
                 double ws = p;
@@ -286,8 +287,9 @@ __global__ __launch_bounds__(kRun) void sample_plain_kernel(SampleArgs a) {
                 if (target < before + s_sum[wave]) {
                     double run = before;
                     for (int e = 0; e < 64; e++) {
-                        run += readlane_d(p, e);
-                        if (target < run) {
+                        const double pe = readlane_d(p, e);
+                        run += pe;
+                        if (target < run && pe > 0.0) {
                             const int at = (r0 + c) * kRun + wave * 64 + e;
                             if (lane == 0 && at < a.n) atomicMin(&s_token, at);
                             break;
@@ -301,6 +303,20 @@ __global__ __launch_bounds__(kRun) void sample_plain_kernel(SampleArgs a) {
                 }
             }
             acc = next;
+        }
+    }
+    // sums left short up to the end: the last token of a probability (none: the last)
+    for (int r = runs - 1; r >= 0 && !done; r--) {
+        if (!(part_sum(a.part + 3 * r, top, t) > 0.0)) continue;  // (uniform)
+        const int i = r * kRun + tid;
+        __syncthreads();
+        if (tid == 0) s_token = -1;
+        __syncthreads();
+        if (i < a.n && prob(a.logits[i], top, t) > 0.0) atomicMax(&s_token, i);
+        __syncthreads();
+        if (s_token >= 0) {
+            token = s_token;
+            done = true;
         }
     }
     if (tid == 0) {
