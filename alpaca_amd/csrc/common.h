@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "per_device.h"
+
 typedef _Float16 f16;
 typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 f16x4 __attribute__((ext_vector_type(4)));
@@ -225,6 +227,15 @@ hipError_t launch_embed(const int32_t* tokens, int count, const DevMatrix& table
 hipError_t launch_dequant(const DevMatrix& m, float* out, hipStream_t st);
 // f16 copy of a matrix (the prefill weight cache): f16(d*q) per weight, cols % 8 == 0.
 hipError_t launch_dequant_f16(const DevMatrix& m, f16* out, hipStream_t st);
+// Lets a kernel have the CU's whole LDS as dynamic memory on the current device
+// (`once`: the kernel's own; the limit is an attribute of each device's copy).
+inline hipError_t allow_whole_lds(OncePerDevice& once, const void* kernel) {
+    int dev = -1;
+    if (hipError_t e = hipGetDevice(&dev)) return e;
+    return (hipError_t)once(dev, [&] {
+        return (int)hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10);
+    });
+}
 // Greedy arg-max.  Writes the token to *chain_token and emitted[slot] (slot =
 // *pos_dev when pos_dev is set, which is then advanced by one).
 // Sampler.sample for a draw u (kernels_sample.hip): *out the token, *status 1

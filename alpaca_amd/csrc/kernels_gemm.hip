@@ -647,9 +647,8 @@ hipError_t run_f32_rows(const GemmF32Args& a, hipStream_t st) {
         const int nw = f32_waves(a.w.cols / 32);
         const size_t lds = (size_t)2 * nw * (MODE == GEMM_SWIGLU ? 2 : 1) * MT * 64 * 4;
         auto* kernel = gemm_f32_kernel<FMT, MODE, MT>;
-        static const hipError_t attr =
-            hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10);
-        if (attr != hipSuccess) return attr;
+        static OncePerDevice once;
+        if (hipError_t e = allow_whole_lds(once, (const void*)kernel)) return e;
         kernel<<<dim3((a.M + MT - 1) / MT, cols), 64 * nw, lds, st>>>(a);
     }
     return hipGetLastError();

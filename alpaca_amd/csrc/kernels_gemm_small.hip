@@ -508,9 +508,8 @@ hipError_t run_small(const SmallArgs& a, hipStream_t st) {
     const int tiles = ((a.M + 16 * TM - 1) / (16 * TM)) * ((a.w.rows + 16 * TN - 1) / (16 * TN));
     const size_t lds = small_lds<FMT, MODE, TM, TN, NW, D, NV, F32>(a.w.cols);
     auto* kernel = small_gemm_kernel<FMT, MODE, TM, TN, NW, D, NV, F32>;
-    static const hipError_t attr =
-        hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 << 10);
-    if (attr != hipSuccess) return attr;
+    static OncePerDevice once;
+    if (hipError_t e = allow_whole_lds(once, (const void*)kernel)) return e;
     kernel<<<tiles, 64 * NW, lds, st>>>(a);
     return hipGetLastError();
 }
