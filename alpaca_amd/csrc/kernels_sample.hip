@@ -284,7 +284,7 @@ __global__ __launch_bounds__(kRun) void sample_plain_kernel(SampleArgs a) {
                 __syncthreads();
                 double before = acc;
                 for (int w = 0; w < wave; w++) before += s_sum[w];
-                if (target < before + s_sum[wave]) {
+                if (s_sum[wave] > 0.0 && target < before + s_sum[wave]) {
                     double run = before;
                     for (int e = 0; e < 64; e++) {
                         const double pe = readlane_d(p, e);
@@ -306,7 +306,7 @@ __global__ __launch_bounds__(kRun) void sample_plain_kernel(SampleArgs a) {
         }
     }
     // sums left short up to the end: the last token of a probability (none: the last)
-    for (int r = runs - 1; r >= 0 && !done; r--) {
+    for (int r = total > 0.0 ? runs - 1 : -1; r >= 0 && !done; r--) {
         if (!(part_sum(a.part + 3 * r, top, t) > 0.0)) continue;  // (uniform)
         const int i = r * kRun + tid;
         __syncthreads();
@@ -435,19 +435,29 @@ __global__ __launch_bounds__(kST) void sample_kernel(SampleArgs a) {
 
     // The next candidates by threshold, at least min(want, left) of them where
     // that fits a window: their number, their composites unsorted in s_win; 0
-    // where no threshold separates 1 to kWin of them.
+    // where no threshold separates 1 to kWin of them.  A search in vain is 24
+    // steps, so the ties with pv that are left are counted before it where the
+    // last window was taken by radix select, which may have ended among more of
+    // them than a window holds, and after six steps in vain.
+    bool in_ties = false;  // the last window was taken by radix select
     auto threshold_window = [&](int want) -> int {
         if (!loaded) load();
         const int soft = min(kWin, max(64, 4 * want));  // a few more steps are cheaper than sorting many more
         const float pv = have_prev ? key_value((uint32_t)(prev >> 32)) : bm;
+        if (!(pv < INFINITY)) return 0;  // (no distance below an infinity)
         const uint32_t pi = (uint32_t)prev;
         float lo = 0.f, hi = 0.f;  // distances known to admit too few, too many (0: none yet)
         float d = width > 0.f ? width : 0.5f;
         int best = 0;
         float best_thr = 0.f;
-        for (int step = 0; step < 24; step++) {
-            const float thr = pv - d;
+        for (int step = in_ties ? -1 : 0; step < 24; step++) {
+            const bool ties = step == -1 || (step == 6 && !best);
+            const float thr = ties ? pv : pv - d;
             const int c = count_to(thr);
+            if (ties) {
+                if (c > kWin) return 0;
+                continue;
+            }
             const bool fits = c >= 1 && c <= kWin;
             if (fits && (!best || (best < want ? c > best : c >= want && c < best))) {
                 best = c;
@@ -553,6 +563,7 @@ __global__ __launch_bounds__(kST) void sample_kernel(SampleArgs a) {
             __syncthreads();
         }
         if (!c) c = threshold_window(min(min(want, kWin / 2), n - produced));
+        in_ties = !c;
         if (!c) {
             c = min(kWin, n - produced);
             radix_window(c);
