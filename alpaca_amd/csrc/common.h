@@ -196,6 +196,30 @@ __device__ __forceinline__ float lane_sum(float v) { return lane_reduce<N>(v, Ad
 __device__ __forceinline__ float wave_sum(float v) { return lane_reduce<64>(v, AddOp()); }
 __device__ __forceinline__ float wave_max(float v) { return lane_reduce<64>(v, MaxOp()); }
 
+// CPUOps.rmsNorm (CPUOps.swift:144-159) of a row held by a wave, V float4 a lane
+// (zeros past the row's end): the factor, and a group of four scaled.
+template <int V>
+__device__ __forceinline__ float rms_scale(const float4 (&v)[V], int dim, float eps) {
+    float ss = 0.f;
+#pragma unroll
+    for (int k = 0; k < V; k++) {
+        ss += v[k].x * v[k].x;
+        ss += v[k].y * v[k].y;
+        ss += v[k].z * v[k].z;
+        ss += v[k].w * v[k].w;
+    }
+    return 1.0f / sqrtf(wave_sum(ss) / (float)dim + eps);
+}
+__device__ __forceinline__ float4 rms_scaled(float4 v, float scale, float4 gain) {
+    return {(v.x * scale) * gain.x, (v.y * scale) * gain.y, (v.z * scale) * gain.z, (v.w * scale) * gain.w};
+}
+// Four values as f16, and the second terms: f16 of what those leave.
+__device__ __forceinline__ f16x4 f16_first(float4 y) { return {(f16)y.x, (f16)y.y, (f16)y.z, (f16)y.w}; }
+__device__ __forceinline__ f16x4 f16_second(float4 y, f16x4 hi) {
+    return {(f16)(y.x - (float)hi[0]), (f16)(y.y - (float)hi[1]), (f16)(y.z - (float)hi[2]),
+            (f16)(y.w - (float)hi[3])};
+}
+
 // Block-wide sum over blockDim.x (a multiple of 64, at most 1024) threads.
 __device__ __forceinline__ float block_sum(float v, float* red /* >= 16 floats of LDS */) {
     v = wave_sum(v);
@@ -223,6 +247,8 @@ hipError_t launch_f32_to_f16(const float* x, f16* out, f16* out_lo, int64_t n, h
 // With out_f16_lo, the second term is written for rows >= lo_row0.
 hipError_t launch_rmsnorm(const float* x, const float* w, float* out_f32, f16* out_f16, f16* out_f16_lo, int rows,
                           int dim, float eps, hipStream_t st, int lo_row0 = 0);
+// Compute units of the current device (256 if that cannot be found out).
+int device_cus();
 hipError_t launch_embed(const int32_t* tokens, int count, const DevMatrix& table, float* out, hipStream_t st);
 hipError_t launch_dequant(const DevMatrix& m, float* out, hipStream_t st);
 // f16 copy of a matrix (the prefill weight cache): f16(d*q) per weight, cols % 8 == 0.

@@ -8,6 +8,13 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 __device__ __forceinline__ h2 as_h2(uint32_t v) { return __builtin_bit_cast(h2, v); }
 __device__ __forceinline__ uint32_t as_u32(h2 v) { return __builtin_bit_cast(uint32_t, v); }
 
+// XOR swizzles of the 16-byte chunks of an LDS tile's rows, so that the rows of a
+// fragment read fall in distinct bank groups: f16 activations or weights (128 B
+// rows of 64 values), Q8_0 quants (64 B) and Q4_0 quants (32 B).
+__device__ __forceinline__ int swz_a(int r) { return (r & 7) ^ ((r >> 1) & 4); }
+__device__ __forceinline__ int swz_q8(int r) { return (r >> 2) & 3; }
+__device__ __forceinline__ int swz_q4(int r) { return (r >> 3) & 1; }
+
 // 4 signed bytes -> 2 dwords holding the 4 quants as f16 pairs (exact).
 __device__ __forceinline__ void int8x4_to_f16(uint32_t w, uint32_t& o0, uint32_t& o1) {
     const uint32_t u = w ^ 0x80808080u;  // q + 128 in each byte

@@ -1326,16 +1326,8 @@ hipError_t launch_attention_merge(const float* partials, int heads, int hd, int 
 // 4,176 positions) 1,056 workgroups and 256-position splits 544; 288-position
 // splits give 480.
 int attention_decode_session_split_len(int capacity, int heads, int kv_heads) {
-    static int cus[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-    if (!cus[dev]) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
-        cus[dev] = n;
-    }
     const int most = kv_heads > 0 && heads / kv_heads <= 2 ? kMaxSplitLenWide : kMaxSplitLen;
-    const int64_t target = 2 * (int64_t)cus[dev];
+    const int64_t target = 2 * (int64_t)device_cus();
     int l = (int)(((int64_t)capacity * kv_heads + target - 1) / target);
     const int fewest = (capacity + 63) / 64;  // at most 64 splits
     l = std::max(std::max(l, fewest), 64);

@@ -654,8 +654,6 @@ hipError_t run_f32_rows(const GemmF32Args& a, hipStream_t st) {
     return hipGetLastError();
 }
 
-int device_cus();
-
 // The kernels against each other.  A 64x64 tile walks K on one thread per 16
 // outputs, 0.14-0.15 us a column of K (0.25 with SwiGLU's two matrices) however
 // few rows there are, and runs at 20-23 products a ns once it has covered the chip
@@ -769,10 +767,6 @@ hipError_t launch_gemm_f32(const float* x, int ldx, int m, const DevMatrix& w, c
 namespace {
 
 constexpr int DBK = 64;  // K per stage
-
-__device__ __forceinline__ int swz_a(int r) { return (r & 7) ^ ((r >> 1) & 4); }
-__device__ __forceinline__ int swz_q8(int r) { return (r >> 2) & 3; }
-__device__ __forceinline__ int swz_q4(int r) { return (r >> 3) & 1; }
 
 // Byte layout of one stage buffer: A rows (the second term's A rows after
 // them, two-term kernels), then each matrix's weight rows, then each matrix's
@@ -1377,19 +1371,6 @@ int forced_tile() {
     if (!std::strcmp(e, "64x64")) return 5;
     if (!std::strcmp(e, "64x64k2")) return 9;
     return 0;
-}
-
-// Compute units of the current device (cached per device id).
-int device_cus() {
-    static int cus[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (!cus[dev]) {
-        int n = 0;
-        hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev);
-        cus[dev] = n > 0 ? n : 256;
-    }
-    return cus[dev];
 }
 
 // Resident workgroups per CU of one instantiation (registers and LDS as

@@ -65,10 +65,6 @@ struct SmallArgs {
     QkvRope qkv;
 };
 
-__device__ __forceinline__ int swz_a(int r) { return (r & 7) ^ ((r >> 1) & 4); }
-__device__ __forceinline__ int swz_q8(int r) { return (r >> 2) & 3; }
-__device__ __forceinline__ int swz_q4(int r) { return (r >> 3) & 1; }
-
 constexpr int SK = 64;  // K per stage (two quant blocks)
 constexpr int kNormV = 4;  // float4 per lane of a normalised row (K <= 1,024)
 
@@ -367,33 +363,19 @@ __global__ __launch_bounds__(64 * NW) void small_gemm_kernel(SmallArgs p) {
             for (int q = 0; q < RPW; q++) {
                 const int row = wave + q * NW;
                 if (row >= 16 * TM) break;
-                float ss = 0.f;
-#pragma unroll
-                for (int k = 0; k < NV; k++) {
-                    ss += v[q][k].x * v[q][k].x;
-                    ss += v[q][k].y * v[q][k].y;
-                    ss += v[q][k].z * v[q][k].z;
-                    ss += v[q][k].w * v[q][k].w;
-                }
-                ss = wave_sum(ss);
-                const float scale = 1.0f / sqrtf(ss / (float)K + p.in.eps);
+                const float scale = rms_scale(v[q], K, p.in.eps);
 #pragma unroll
                 for (int k = 0; k < NV; k++) {
                     const int i = lane + 64 * k;
                     if (i >= n4) break;
-                    const float4 gn = gv[k];
-                    const float4 yv = {(v[q][k].x * scale) * gn.x, (v[q][k].y * scale) * gn.y,
-                                       (v[q][k].z * scale) * gn.z, (v[q][k].w * scale) * gn.w};
+                    const float4 yv = rms_scaled(v[q][k], scale, gv[k]);
                     if constexpr (F32) {
                         *(f32x4*)(rows + row * pitch + 16 * i) = f32x4{yv.x, yv.y, yv.z, yv.w};
                         continue;
                     }
-                    const f16x4 hi = {(f16)yv.x, (f16)yv.y, (f16)yv.z, (f16)yv.w};
+                    const f16x4 hi = f16_first(yv);
                     *(f16x4*)(rows + row * pitch + 8 * i) = hi;
-                    if constexpr (TT)
-                        *(f16x4*)(rows + (16 * TM + row) * pitch + 8 * i) =
-                            f16x4{(f16)(yv.x - (float)hi[0]), (f16)(yv.y - (float)hi[1]), (f16)(yv.z - (float)hi[2]),
-                                  (f16)(yv.w - (float)hi[3])};
+                    if constexpr (TT) *(f16x4*)(rows + (16 * TM + row) * pitch + 8 * i) = f16_second(yv, hi);
                 }
             }
             __syncthreads();
@@ -552,18 +534,6 @@ hipError_t run_input(int mode, int family, const SmallArgs& a, hipStream_t st) {
     if (a.in.f32)
         return norm ? run_mode<FMT, kNormV, true>(mode, family, a, st) : run_mode<FMT, 0, true>(mode, family, a, st);
     return norm ? run_mode<FMT, kNormV, false>(mode, family, a, st) : run_mode<FMT, 0, false>(mode, family, a, st);
-}
-
-int device_cus() {
-    static int cus[64] = {0};
-    int dev = 0;
-    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
-    if (!cus[dev]) {
-        int n = 0;
-        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
-        cus[dev] = n;
-    }
-    return cus[dev];
 }
 
 }  // namespace

@@ -7,6 +7,8 @@
 #include <float.h>
 #include <limits.h>
 
+#include <atomic>
+
 namespace {
 
 constexpr int kBlock = 256;
@@ -78,37 +80,23 @@ __global__ __launch_bounds__(kBlock) void rmsnorm_rows_kernel(const float* x, co
     const float4* wr = (const float4*)w;
     // the gains load with the row, not after the reduction
     float4 v[kNormV4], gv[kNormV4];
-    float ss = 0.f;
 #pragma unroll
     for (int k = 0; k < kNormV4; k++) {
         const int i = lane + 64 * k;
         v[k] = i < n4 ? xr[i] : float4{0.f, 0.f, 0.f, 0.f};
         gv[k] = i < n4 ? wr[i] : float4{0.f, 0.f, 0.f, 0.f};
     }
-#pragma unroll
-    for (int k = 0; k < kNormV4; k++) {
-        ss += v[k].x * v[k].x;
-        ss += v[k].y * v[k].y;
-        ss += v[k].z * v[k].z;
-        ss += v[k].w * v[k].w;
-    }
-    ss = wave_sum(ss);
-    const float scale = 1.0f / sqrtf(ss / (float)dim + eps);
+    const float scale = rms_scale(v, dim, eps);
 #pragma unroll
     for (int k = 0; k < kNormV4; k++) {
         const int i = lane + 64 * k;
         if (i >= n4) break;
-        const float4 g = gv[k];
-        const float4 y = {(v[k].x * scale) * g.x, (v[k].y * scale) * g.y, (v[k].z * scale) * g.z,
-                          (v[k].w * scale) * g.w};
+        const float4 y = rms_scaled(v[k], scale, gv[k]);
         if (of) ((float4*)(of + (int64_t)row * dim))[i] = y;
         if (oh) {
-            typedef _Float16 h4 __attribute__((ext_vector_type(4)));
-            const h4 hi = {(f16)y.x, (f16)y.y, (f16)y.z, (f16)y.w};
-            ((h4*)(oh + (int64_t)row * dim))[i] = hi;
-            if (ol)
-                ((h4*)(ol + (int64_t)row * dim))[i] = h4{(f16)(y.x - (float)hi[0]), (f16)(y.y - (float)hi[1]),
-                                                         (f16)(y.z - (float)hi[2]), (f16)(y.w - (float)hi[3])};
+            const f16x4 hi = f16_first(y);
+            ((f16x4*)(oh + (int64_t)row * dim))[i] = hi;
+            if (ol) ((f16x4*)(ol + (int64_t)row * dim))[i] = f16_second(y, hi);
         }
     }
 }
@@ -292,6 +280,17 @@ hipError_t launch_rmsnorm(const float* x, const float* w, float* of, f16* oh, f1
     if (vec) rmsnorm_rows_kernel<<<(rows + 3) / 4, kBlock, 0, st>>>(x, w, of, oh, ol, rows, dim, eps, lo_row0);
     else rmsnorm_kernel<<<rows, kBlock, 0, st>>>(x, w, of, oh, ol, dim, eps, lo_row0);
     return hipGetLastError();
+}
+int device_cus() {
+    static std::atomic<int> cus[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 256;
+    int n = cus[dev].load(std::memory_order_relaxed);
+    if (!n) {
+        if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || n < 1) n = 256;
+        cus[dev].store(n, std::memory_order_relaxed);
+    }
+    return n;
 }
 hipError_t launch_embed(const int32_t* tokens, int count, const DevMatrix& table, float* out, hipStream_t st) {
     if (count > 0) embed_kernel<<<count, kBlock, 0, st>>>(tokens, table, out);
