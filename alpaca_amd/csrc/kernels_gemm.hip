@@ -1410,9 +1410,9 @@ hipError_t pick_dgemm(const GemmArgs& a, hipStream_t st) {
     // 64x64 (64x32 per matrix), two per SIMD, so that one wave's VALU work
     // (block scaling, quant conversion) issues while the other's MFMAs run:
     // at the 1.7B shape 4-7% faster than four waves of 64x128.  Single-term
-    // activations stay on the narrower tiles, where the wide ones measured
-    // slower: 128x64 tiles (two LDS stages) while their grid fits in one round
-    // of the workgroups the device holds at once, else 128x128.  With two
+    // activations never take 128x256, where they measured slower: 64x64 on small
+    // grids (below), else 128x64 tiles (two LDS stages) while their grid fits in
+    // one round of the workgroups the device holds at once, else 128x128.  With two
     // terms, small grids (at most 1.6 tiles of 128x64 per CU, 3 for SwiGLU,
     // whose 128x64 tiles run one per CU) take 64x64 tiles (two LDS stages,
     // three workgroups per CU with quantised weights): at the 135M shape over

@@ -541,8 +541,11 @@ hipError_t run_input(int mode, int family, const SmallArgs& a, hipStream_t st) {
 // The rule: the smallest tile whose grid is at most one workgroup per CU, or
 // none (the pipelined tiles of kernels_gemm.hip, which share operands better,
 // take the grids past that).  Every family costs about a launch, one memory
-// round trip and its tile's bytes, so the smallest wins while each CU runs one;
-// a second round costs as much as the first.  Two activation terms, Q8_0,
+// round trip and its tile's bytes, so the smallest wins while each CU runs one.
+// A second workgroup on some CUs takes most of that again: past the line the
+// 32x64 tiles lose up to 22% or, where K is long and the pipelined tiles pay its
+// length in stages, gain up to 8% (the bracketed figures), so the line stays at
+// the last grid that always gains.  Two activation terms, Q8_0,
 // weights from HBM, us per launch (pipelined tiles -> these):
 //   135M shape     QKV          gate+up       down         Wo
 //    11 rows    7.8 -> 3.6   10.0 -> 3.7   11.7 -> 3.9   6.7 -> 3.3

@@ -1914,7 +1914,8 @@ static int check_sampling(float temperature, int top_k, float top_p, double u) {
     return AHIP_OK;
 }
 
-// One sample_kernel launch over device logits; the token comes back through a small copy.
+// Two or three launches over device logits (launch_sample; one for the arg-max of up to 1,024); the
+// token comes back through a small copy.
 static int run_sample(const float* dlogits, int n, float temperature, int top_k, float top_p, double u,
                       DevBuf& idx, DevBuf& prob, DevBuf& out, hipStream_t st, int32_t* token) {
     if (!idx.p)

@@ -53,7 +53,9 @@ typedef enum { AHIP_KV_F16 = 0, AHIP_KV_F32 = 1 } ahip_kv_precision;
  * logits stay within 2e-3 + 1e-3 relative of the CPU reference at every
  * benchmark configuration; fast_f16 = the same MFMA kernels with one f16 term
  * per activation (the reference's fast-path numerics class: half the MFMA
- * work, 2^-11 relative input rounding). */
+ * work, 2^-11 relative input rounding).  Both modes' prompts of 16 tokens and
+ * more need activations inside f16's range (65,504); shorter calls keep float32
+ * operands. */
 typedef enum { AHIP_GEMM_EXACT = 0, AHIP_GEMM_FAST = 1, AHIP_GEMM_FAST_F16 = 2 } ahip_gemm_precision;
 
 /* LlamaConfig, Sources/AlpacaCore/Transformer/LlamaConfig.swift:8-20. */

@@ -10,7 +10,7 @@ import oracle.oracle as orc
 from alpaca_amd import synth
 from alpaca_amd.model import HIPLlamaModel
 from alpaca_amd.tensor import F16, F32, Q4_0, Q8_0, encode
-from tests.helpers import assert_close
+from tests.helpers import assert_close, env
 from tests.test_gpu_kernels import FORMATS
 from tests.test_gpu_model import built, oracle_cfg
 
@@ -127,4 +127,19 @@ def test_short_calls_of_every_form(hip_ctx, hidden, heads, kv, hd, ffn, dt):
     for part in (tokens[:2], tokens[2:13], tokens[13:28], tokens[28:33]):
         want = exact.forward(part)
         assert_close(fast.forward(part), want, 2.5e-4 * float(np.abs(want).max()), 0.0, f"{len(part)} tokens")
+    model.close()
+
+
+@pytest.mark.parametrize("hd", [32, 64, 128])
+def test_short_calls_rotate_and_append_as_the_separate_kernel(hip_ctx, hd):
+    """RoPE and the KV append in the GEMM's epilogue against the GEMM and then the RoPE kernel: the same
+    products and roundings, so the same bits, in the logits and in the decode step over the cache."""
+    spec = replace(SPEC, name=f"rope-{hd}", config=replace(SPEC.config, head_dim=hd, head_count=4, kv_head_count=2))
+    model = HIPLlamaModel(hip_ctx, spec.config, built(spec))
+    fused = model.make_session()
+    with env(ALPACA_HIP_FUSE_QKV_ROPE=0):
+        apart = model.make_session()
+    tokens = synth.prompt_tokens(spec, 40)
+    for part in (tokens[:15], tokens[15:17], tokens[17:28], tokens[28:29]):
+        assert np.array_equal(fused.forward(part).view(np.uint32), apart.forward(part).view(np.uint32)), len(part)
     model.close()

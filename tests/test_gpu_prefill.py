@@ -140,7 +140,8 @@ def test_two_stream_prefill_matches_one_stream(hip_ctx, spec, prec, rows):
     bit can then round to the neighbouring f16 (2^-11 relative) in the one-term
     rows, so the runs agree to 2.5e-4 of the peak, and each is held to the
     CPU oracle at full size by the C1P workload test.  (One-term activations
-    throughout, fast-f16, never take the two-K-set tiles, and agree to 1e-5.)
+    throughout, fast-f16, take two K sets and the few-row kernel only below 768
+    rows, the shortest half of a split prompt, and agree to 1e-5.)
     Cases: a 1600-token
     chunk (halves of 768 and 832 rows, just past the 1,536-token threshold),
     one 3100-token chunk (uneven halves), then a 4300-token prompt over chunks
