@@ -28,7 +28,8 @@
 //
 // F32 (calls of 2 to 15 tokens): float32 activations without loss.  A float32 is
 // the exact sum of three bf16 terms (24 significant bits in three times 8, the
-// exponent range the same), a quant or nibble is one and an f16 weight two, so
+// exponent range the same; below 2^-102 the last ones are subnormal and may be
+// lost, 2^-126 at most), a quant or nibble is one and an f16 weight two, so
 // bf16 MFMA products of the terms are the float32 products themselves, summed in
 // float32, smallest terms first.  The rows stay float32 in HBM and LDS (the bytes
 // of two f16 terms) and a lane takes a fragment apart as it reads it: with K split
@@ -111,7 +112,8 @@ __device__ __forceinline__ bf16x8 as_bf16x8(const uint32_t (&o)[4]) {
     return __builtin_bit_cast(bf16x8, make_uint4(o[0], o[1], o[2], o[3]));
 }
 // Eight floats as N bf16 terms, largest first: each the top half of what the ones
-// before it leave (exact differences; three hold every float32, two every f16).
+// before it leave (exact differences; three hold a float32 from 2^-102 on, two
+// every f16).
 template <int N>
 __device__ __forceinline__ void bf16_split(float (&x)[8], bf16x8 (&t)[N]) {
 #pragma unroll

@@ -1666,7 +1666,7 @@ static int encode_chunk(ahip_session* s, const int32_t* dtok, int n, int pos, bo
                 }
                 s->stage(stage);
                 if (few && gemm_small_takes(rows, n, w, up)) {
-                    roped = mode == GEMM_QKV_ROPE;
+                    if (mode == GEMM_QKV_ROPE) roped = true;
                     return launch_gemm_small(rows, n, w, up, y, nullptr, nullptr, ldy, mode, &o, st, 0, 0);
                 }
                 return launch_gemm_f32(rows.xf, w.cols, n, w, up, y, ldy, mode == GEMM_QKV_ROPE ? GEMM_STORE : mode, st);

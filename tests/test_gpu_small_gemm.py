@@ -6,7 +6,9 @@ Against the oracle at the shapes where each tile is chosen, with partial tiles
 in both directions, and against the pipelined tiles (ALPACA_HIP_GEMM_TILE
 forces one, read per launch) through sessions, where the same float32 products
 are summed in another order: 1e-5 of the logit peak, as between the pipelined
-tiles and their two-K-set form.
+tiles and their two-K-set form.  (Calls of 2 to 15 tokens have no pipelined form:
+there the override changes nothing, and what they are held to is the float32
+kernels, here and in test_gpu_few_rows.)
 """
 from dataclasses import replace
 
