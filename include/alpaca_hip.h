@@ -130,7 +130,8 @@ int ahip_model_weight_bytes(const ahip_model* model, int64_t* bytes);
  * with prefill_weight_cache set, every quantised layer projection also gets an
  * f16 copy (each weight d*q rounded once to f16, buildPrefillCache :97-120)
  * that the fast prefill GEMMs multiply by instead of dequantising blocks;
- * decode and the exact prefill keep using the quantised weights.  0 when not
+ * decode, calls of 2 to 15 tokens and the exact prefill keep using the
+ * quantised weights.  0 when not
  * requested or when the layers are already F16. */
 int ahip_model_prefill_cache_bytes(const ahip_model* model, int64_t* bytes);
 
